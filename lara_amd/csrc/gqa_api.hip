@@ -396,7 +396,7 @@ int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_p
         r.scale_bits = sb;
         r.out = (uint16_t*)o;
         r.lse = lse;
-        HIP_TRY(launch_rtl_transaction(c->cfg.head_dim, r, timed(c, GQA_TIMER_PREFILL, s)));
+        HIP_TRY(launch_rtl_transaction(c->cfg.head_dim, r, c->n_cu, timed(c, GQA_TIMER_PREFILL, s)));
         c->last_prefill_kernel = 0;
         c->last_prefill_segs = 0;
         return GQA_OK;

@@ -189,8 +189,9 @@ struct RtlArgs {
     uint32_t scale_bits;    // fp32 bits of the score scale (the board's INV_SQRT_D_FP32)
     uint16_t* out;          // [H_q][q_len][D] bf16
     float* lse;             // [H_q][q_len] or nullptr
+    int32_t pair_tiles;     // set by the launch: short row tiles beside long ones
 };
-hipError_t launch_rtl_transaction(int head_dim, const RtlArgs& a, const Launch& l);
+hipError_t launch_rtl_transaction(int head_dim, const RtlArgs& a, int n_cu, const Launch& l);
 
 // Splits of a sequence of L attended keys cut into `chunk`-key splits: a last split of at most
 // chunk/4 keys is folded into the one before it (no work-group is left with a handful of keys, such

@@ -113,3 +113,58 @@ def test_board_functional_matrix_on_board_format_cases(tmp_path):
     files["expected_o"][3, 1, 7] ^= 1
     np.savez(bad / src.name, **files)
     assert board_matrix.main(["--cases", str(bad), "--output-dir", str(tmp_path / "bad")]) == 1
+
+
+def _extreme_inputs(kind, L, d):
+    """Inputs that push one step of the kernel off native arithmetic (or to the edge of it)."""
+    rng = np.random.default_rng(2400 + L + d)
+    q, k, v = (bf16_normal(rng, (h, L, d)) for h in (4, 2, 2))
+    tiny, huge = np.uint16([0x2380, 0xA3FF, 0x237F, 0x0000]), np.uint16([0x507F, 0xD07F, 0x5080, 0x8000])
+    if kind == "wild key":  # one K row outside the native range, in the second 64 keys where there is one
+        k[1, L - 1, 3] = 0x0001
+    elif kind == "wild query":
+        q[2, L // 2, :4] = np.uint16([0x7F80, 0x7F00, 0x0080, 0xFF80])
+    elif kind == "wild value":  # NaN and infinities in V, then ordinary rows
+        v[0, L // 3, :3] = np.uint16([0x7FC0, 0x7F80, 0xFF80])
+    elif kind == "range edges":  # words at both ends of the native range, and just outside it
+        q[:, :, ::5], k[:, :, ::7] = rng.choice(tiny, (4, L, len(range(0, d, 5)))), rng.choice(huge, (2, L, len(range(0, d, 7))))
+        v[:, :, ::3] = rng.choice(np.concatenate([tiny, huge]), (2, L, len(range(0, d, 3))))
+    elif kind == "native edges":  # the same ends, nothing outside: subnormal remainders of cancelling sums
+        q[:], k[:] = rng.choice(tiny[:2], q.shape), rng.choice(np.uint16([0x2380, 0xA380, 0x5000, 0xD000]), k.shape)
+    elif kind == "zero signs":  # O elements that are zero for a while or throughout, of either sign
+        v[:, :, : d // 2] = rng.choice(np.uint16([0x0000, 0x8000]), (2, L, d // 2))
+        v[:, : L // 2, d // 2:] = 0x8000
+    elif kind == "rising scores":  # each sub-block's max passes the last by more than 8: corr = 0
+        k[:] = 0x3F80
+        k[:, :, 0] = bf16_normal(rng, (2, L)) & 0x7FFF
+        q[:] = 0x0000
+        q[:, :, 1] = 0x42C8
+        k[:, :, 1] = (np.arange(L) * 2.0).astype(np.float32).view(np.uint32) >> 16
+    return q, k, v
+
+
+@pytest.mark.parametrize("kind", ["wild key", "wild query", "wild value", "range edges", "native edges", "zero signs",
+                                  "rising scores", "subnormal scores"])
+@pytest.mark.parametrize("L,d", [(79, 128), (273, 64)])
+def test_kv260_mode_off_native_arithmetic(kind, L, d):
+    q, k, v = _extreme_inputs(kind, L, d)
+    scale = 2.0 ** -128 if kind == "subnormal scores" else None
+    for causal, qb, kb in ((True, 0, 0), (True, 0, 21), (False, 0, 0)):
+        print(f"[kv260] {kind} L={L} d={d} causal={causal} kv_pos_base={kb}", flush=True)
+        with AttentionAccelerator(n_q_heads=4, n_kv_heads=2, head_dim=d, max_seq_len=L, scale=scale,
+                                  numerics="kv260") as acc:
+            out = acc.run_attention(q, k, v, q_pos_base=qb, kv_pos_base=kb, causal=causal)
+            want, _, _ = rtl.attention(q, k, v, causal=causal, q_pos_base=qb, kv_pos_base=kb, scale=acc.scale)
+        mism = np.argwhere(out != want)
+        assert mism.size == 0, f"{len(mism)} mismatching words, first at {tuple(mism[0])}"
+
+
+@pytest.mark.parametrize("L", [15, 17, 31, 63, 65, 255, 256, 257, 497])
+def test_kv260_mode_span_edges(L):
+    """Lengths around the 16-key sub-blocks, 32-row tiles, 64-key waves and 256-key passes."""
+    rng = np.random.default_rng(2500 + L)
+    q, k, v = (bf16_normal(rng, (h, L, 128)) for h in (4, 2, 2))
+    for causal in (True, False):
+        out, want = run_both(q, k, v, causal=causal, qb=0, kb=0)
+        mism = np.argwhere(out != want)
+        assert mism.size == 0, f"{len(mism)} mismatching words, first at {tuple(mism[0])}"
