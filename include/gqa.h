@@ -339,6 +339,9 @@ int gqa_decode_append_noalloc(const gqa_config* cfg, void* k_cache, void* v_cach
  * times them on the caller's operands (each run four times, the stream synchronised once per
  * algorithm: a few ms, once) and later calls use the fastest, while calls under a capture use the
  * best-ranked until such a call has run.  The context keeps the last 8 shapes.
+ * Calls of up to 16 tokens (8 at hidden 8192) with hidden 1024, 2048, 4096 or 8192, 16-byte aligned
+ * operands and outputs apart from them run as one launch of the library's own instead (no workspace, nothing
+ * tuned), timed as the projection: the stages' other two times are then about zero.
  * gqa_layer_times returns the device time in us of
  * the RMSNorm, projection and RoPE stages (n <= 3; synchronises) of the last gqa_submit_layer
  * call (GQA_ERR_NO_TRANSACTION when there is none); gqa_layer_qkv_device calls made while

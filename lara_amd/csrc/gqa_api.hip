@@ -22,6 +22,7 @@ constexpr int kChunkOptionQuantum = 64;  // GQA_OPT_DECODE_CHUNK: a multiple of 
 constexpr int kMinSplitCap = 256;        // the split workspace holds at least l_cap / this splits
 constexpr int kMaxPrefillSegs = 16;
 constexpr int32_t kMaxRows = 1 << 30;  // max_seq_len / max_q_len limit: row counts rounded up stay in int32
+constexpr double kRopeBase = 10000.0;  // theta_p = 10000^(-2p/D): hw/data/rope_theta.hex for D = 128
 constexpr int kDecodeWavesPerCu = 8;  // split planner target; one split per (sequence, kv head) once that fills the GPU
 
 struct Txn {
@@ -110,6 +111,7 @@ struct gqa_ctx {
     uint8_t* lt_ws = nullptr;      // hipBLASLt workspace of the projection algorithms in use
     size_t lt_ws_bytes = 0;
     hipEvent_t ev_layer[4] = {};
+    float theta[kMaxRopePairs] = {};  // RoPE frequencies
     float layer_us[3] = {};
     bool layer_timed = false;  // ev_layer holds a recorded call
     // Paged cache (gqa_create_paged): k_cache/v_cache are page pools [n_pages][H_kv][P][D], the
@@ -166,6 +168,11 @@ bool rows_backed(const gqa_ctx* c, int b, int64_t row0, int64_t n) {
 }
 
 hipStream_t pick_stream(gqa_ctx* c, void* s) { return s ? (hipStream_t)s : c->stream; }
+
+inline bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return na > 0 && nb > 0 && x < y + nb && y < x + na;
+}
 
 // Device operands the kernels move in 16-byte vectors (Q, appended K/V rows, prefill output)
 // must be 16-byte aligned; nullptr passes (optional operands are checked for presence apart).
@@ -511,8 +518,6 @@ int ensure_buffer(uint8_t** buf, size_t* cap, size_t bytes) {
     return GQA_OK;
 }
 
-constexpr double kRopeBase = 10000.0;  // theta_p = 10000^(-2p/D): hw/data/rope_theta.hex for D = 128
-
 int check_layer_args(const gqa_ctx* c, int32_t b, int32_t n_tokens, int32_t hidden, int32_t q_pos_base,
                      int32_t kv_pos_base, int32_t row0) {
     if (b < 0 || b >= c->cfg.batch) return GQA_ERR_STREAM_DEST;
@@ -632,6 +637,55 @@ int run_layer_qkv(gqa_ctx* c, int32_t b, const void* x, int32_t n_tokens, int32_
                   int32_t kv_pos_base, int32_t row0, int32_t rope, void* q_out, hipStream_t s, bool stage_events) {
     const int D = c->cfg.head_dim, nq = c->cfg.n_q_heads * D, nkv = c->cfg.n_kv_heads * D;
     const int ld = nq + 2 * nkv;
+    RopeArgs ra{};
+    ra.n_tokens = n_tokens;
+    ra.n_q_heads = c->cfg.n_q_heads;
+    ra.n_kv_heads = c->cfg.n_kv_heads;
+    ra.head_dim = D;
+    ra.rope = rope ? 1 : 0;
+    ra.q_out = (uint16_t*)q_out;
+    const size_t seq = c->paged ? 0 : (size_t)b * c->cfg.n_kv_heads * c->l_cap * D;
+    ra.kc = c->k_cache + seq;
+    ra.vc = c->v_cache + seq;
+    ra.block_table = c->paged ? c->table_dev + (size_t)b * c->max_pages : nullptr;
+    ra.page_shift = c->page_shift;
+    ra.l_cap = c->l_cap;
+    ra.row0 = row0;
+    if (stage_events && !c->ev_layer[0])
+        for (int i = 0; i < 4; ++i) HIP_TRY(hipEventCreate(&c->ev_layer[i]));
+    c->layer_timed = false;
+    auto mark = [&](int i) { return stage_events ? hipEventRecord(c->ev_layer[i], s) : hipSuccess; };
+    FewTokensArgs fa{};
+    fa.x = (const uint16_t*)x;
+    fa.gamma = (const uint16_t*)gamma;
+    fa.w[0] = (const uint16_t*)wq;
+    fa.w[1] = (const uint16_t*)wk;
+    fa.w[2] = (const uint16_t*)wv;
+    fa.hidden = hidden;
+    fa.eps = eps;
+    fa.q_pos_base = q_pos_base;
+    fa.kv_pos_base = kv_pos_base;
+    memcpy(fa.theta, c->theta, sizeof(fa.theta));
+    fa.rope = ra;
+    // The one-launch stage reads its inputs while it writes: an output that overlaps one takes the general path.
+    const size_t pool_bytes = kv_words(c) * 2;
+    const struct { const void* p; size_t n; } ins[] = {{x, (size_t)n_tokens * hidden * 2}, {gamma, gamma ? (size_t)hidden * 2 : 0},
+                                                       {wq, (size_t)nq * hidden * 2}, {wk, (size_t)nkv * hidden * 2},
+                                                       {wv, (size_t)nkv * hidden * 2}};
+    bool apart = true;
+    for (const auto& in : ins)
+        apart = apart && !overlaps(in.p, in.n, q_out, (size_t)n_tokens * nq * 2) &&
+                !overlaps(in.p, in.n, c->k_cache, pool_bytes) && !overlaps(in.p, in.n, c->v_cache, pool_bytes);
+    if (apart && few_tokens_supported(fa, c->n_cu)) {
+        // One launch, in the projection's timer slot and between its events.
+        HIP_TRY(mark(0));
+        HIP_TRY(mark(1));
+        HIP_TRY(launch_few_tokens(fa, c->n_cu, stage_events ? Launch{s} : timed(c, GQA_TIMER_PROJECTION, s)));
+        HIP_TRY(mark(2));
+        HIP_TRY(mark(3));
+        c->layer_timed = stage_events;
+        return GQA_OK;
+    }
     const size_t y_bytes = gamma ? ((size_t)n_tokens * hidden * 2 + 255) / 256 * 256 : 0;
     const size_t qkv_bytes = ((size_t)n_tokens * ld * 2 + 255) / 256 * 256;
     const int cs_sets = rope ? (kv_pos_base == q_pos_base ? 1 : 2) : 0;  // RoPE cos/sin table sets
@@ -646,10 +700,6 @@ int run_layer_qkv(gqa_ctx* c, int32_t b, const void* x, int32_t n_tokens, int32_
             return GQA_ERR_HIP;
         }
     }
-    if (stage_events && !c->ev_layer[0])
-        for (int i = 0; i < 4; ++i) HIP_TRY(hipEventCreate(&c->ev_layer[i]));
-    c->layer_timed = false;
-    auto mark = [&](int i) { return stage_events ? hipEventRecord(c->ev_layer[i], s) : hipSuccess; };
     // While profiling (device calls), the projection's hipBLASLt kernels are bracketed by the next
     // event pair of its timer slot; RMSNorm and RoPE have event pairs bound to their launches.
     const Launch proj_events = stage_events ? Launch{s} : timed(c, GQA_TIMER_PROJECTION, s);
@@ -671,7 +721,7 @@ int run_layer_qkv(gqa_ctx* c, int32_t b, const void* x, int32_t n_tokens, int32_
         na.table.n_tokens = n_tokens;
         na.table.q_pos_base = q_pos_base;
         na.table.kv_pos_base = kv_pos_base;
-        for (int p = 0; p < D / 2; ++p) na.table.theta[p] = (float)pow(kRopeBase, -2.0 * p / D);
+        memcpy(na.table.theta, c->theta, sizeof(na.table.theta));
         HIP_TRY(launch_rms_norm(na, stage_events ? Launch{s} : timed(c, GQA_TIMER_NORM, s)));
         if (gamma) src = na.y;
     }
@@ -715,24 +765,10 @@ int run_layer_qkv(gqa_ctx* c, int32_t b, const void* x, int32_t n_tokens, int32_
     }
     if (proj_events.stop) HIP_TRY(hipEventRecord(proj_events.stop, s));
     HIP_TRY(mark(2));
-    RopeArgs ra{};
     ra.qkv = qkv;
     ra.ld = ld;
-    ra.n_tokens = n_tokens;
-    ra.n_q_heads = c->cfg.n_q_heads;
-    ra.n_kv_heads = c->cfg.n_kv_heads;
-    ra.head_dim = D;
-    ra.rope = rope ? 1 : 0;
     ra.cs = cs;
     ra.cs_k_set = cs_sets == 2 ? 1 : 0;
-    ra.q_out = (uint16_t*)q_out;
-    const size_t seq = c->paged ? 0 : (size_t)b * c->cfg.n_kv_heads * c->l_cap * D;
-    ra.kc = c->k_cache + seq;
-    ra.vc = c->v_cache + seq;
-    ra.block_table = c->paged ? c->table_dev + (size_t)b * c->max_pages : nullptr;
-    ra.page_shift = c->page_shift;
-    ra.l_cap = c->l_cap;
-    ra.row0 = row0;
     HIP_TRY(launch_rope_scatter(ra, stage_events ? Launch{s} : timed(c, GQA_TIMER_ROPE, s)));
     HIP_TRY(mark(3));
     c->layer_timed = stage_events;
@@ -795,6 +831,8 @@ int create_ctx(const gqa_config* cfg, int32_t page_size, int32_t n_pages, int32_
     c->scale = k.scale > 0.f ? k.scale : (float)(1.0 / sqrt((double)k.head_dim));
     c->cfg.scale = c->scale;
     c->clock_mhz = prop.clockRate / 1000.0;
+    for (int p = 0; p < std::min(k.head_dim / 2, kMaxRopePairs); ++p)
+        c->theta[p] = (float)pow(kRopeBase, -2.0 * p / k.head_dim);
     if (prop.multiProcessorCount > 0) c->n_cu = prop.multiProcessorCount;
     if (page_size > 0) {
         c->paged = 1;

@@ -271,6 +271,20 @@ struct RopeArgs {
 };
 hipError_t launch_rope_scatter(const RopeArgs& a, const Launch& l);
 
+// RMSNorm (gamma != nullptr), projection, RoPE and scatter of a few tokens in one launch.
+struct FewTokensArgs {
+    const uint16_t* x;      // [n_tokens][hidden] bf16
+    const uint16_t* gamma;  // [hidden] bf16, or nullptr
+    const uint16_t* w[3];   // Wq, Wk, Wv [out][hidden] bf16
+    int hidden;
+    float eps;
+    int q_pos_base, kv_pos_base;
+    float theta[kMaxRopePairs];
+    RopeArgs rope;          // shapes and destinations (qkv, ld and cs unused)
+};
+bool few_tokens_supported(const FewTokensArgs& a, int n_cu);
+hipError_t launch_few_tokens(const FewTokensArgs& a, int n_cu, const Launch& l);
+
 // Streaming-read ceiling probe (probe.hip): reads n_bytes (a multiple of 16) at src with n_wgs
 // 512-thread work-groups, `unroll` (1, 2, 4 or 8) 16-byte nontemporal loads in flight per thread.
 hipError_t launch_stream_read(const void* src, int64_t n_bytes, int n_wgs, int unroll, uint32_t* sink,

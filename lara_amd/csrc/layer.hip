@@ -15,8 +15,13 @@
 //   the sequence's cache rows.
 #include "gqa_internal.h"
 
+#include <algorithm>
+#include <type_traits>
+
 namespace lara {
 namespace {
+
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ float bf16_to_f32(uint32_t w) { return __uint_as_float(w << 16); }
 
@@ -47,9 +52,18 @@ __device__ __forceinline__ u32x4 scale_row(const u32x4& w, const u32x4& g, float
     for (int j = 0; j < 4; ++j) {
         const float lo = __fmul_rn(__fmul_rn(bf16_to_f32(w[j] & 0xFFFFu), inv), bf16_to_f32(g[j] & 0xFFFFu));
         const float hi = __fmul_rn(__fmul_rn(bf16_to_f32(w[j] >> 16), inv), bf16_to_f32(g[j] >> 16));
-        o[j] = (uint32_t)f32_to_bf16_rne(lo) | ((uint32_t)f32_to_bf16_rne(hi) << 16);
+        const bf16x2_t pair = {(__bf16)lo, (__bf16)hi};  // v_cvt_pk_bf16_f32, round to nearest even
+        o[j] = __builtin_bit_cast(uint32_t, pair);
     }
     return o;
+}
+
+// (cos, sin) of the fp32 phase pos * theta, evaluated in double.
+__device__ __forceinline__ float2 rope_cos_sin(int pos, float theta) {
+#pragma clang fp contract(off)
+    double sd, cd;
+    sincos((double)((float)pos * theta), &sd, &cd);
+    return make_float2((float)cd, (float)sd);
 }
 
 // Work-group `wg` (< table_wgs) of a norm launch: one table entry per thread.
@@ -57,12 +71,7 @@ __device__ __forceinline__ void fill_rope_table(const RopeTable& t, int wg) {
     const int i = wg * kNormThreads + threadIdx.x;
     if (i >= t.sets * t.n_tokens * t.pairs) return;
     const int p = i % t.pairs, tok = (i / t.pairs) % t.n_tokens, set = i / (t.pairs * t.n_tokens);
-    {
-#pragma clang fp contract(off)
-        double sd, cd;
-        sincos((double)((float)((set ? t.kv_pos_base : t.q_pos_base) + tok) * t.theta[p]), &sd, &cd);
-        reinterpret_cast<float2*>(t.cs)[i] = make_float2((float)cd, (float)sd);
-    }
+    reinterpret_cast<float2*>(t.cs)[i] = rope_cos_sin((set ? t.kv_pos_base : t.q_pos_base) + tok, t.theta[p]);
 }
 
 // Row-per-wave form for hidden = CPL * 512 (16-byte aligned rows): each wave owns one token
@@ -156,6 +165,22 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(NormArgs a) {
 
 constexpr int kRopeThreads = 256;
 
+// Rotates the pair (x0, x1) of bf16 words; each product and sum is rounded to fp32 on its own.
+__device__ __forceinline__ uint32_t rotate_pair(uint32_t x0w, uint32_t x1w, float c, float s) {
+#pragma clang fp contract(off)
+    const float x0 = bf16_to_f32(x0w), x1 = bf16_to_f32(x1w);
+    const float r0 = x0 * c - x1 * s;
+    const float r1 = x0 * s + x1 * c;
+    return (uint32_t)f32_to_bf16_rne(r0) | ((uint32_t)f32_to_bf16_rne(r1) << 16);
+}
+
+// The K (or V) cache row of kv head g for token t; nullptr where its page is unmapped (nothing to write).
+__device__ __forceinline__ uint16_t* cache_row(const RopeArgs& a, bool is_k, int g, int t) {
+    int64_t r = (int64_t)g * a.l_cap + a.row0 + t;
+    if (a.block_table != nullptr) r = paged_row(a.block_table, a.page_shift, a.n_kv_heads, g, a.row0 + t);
+    return r < 0 ? nullptr : (is_k ? a.kc : a.vc) + (size_t)r * a.head_dim;
+}
+
 // Rotate the four (2p, 2p+1) pairs of one 16-byte chunk of head h by the (cos, sin) values cs
 // (two pairs per float4) and store the chunk at its destination.
 __device__ __forceinline__ void rope_store_chunk(const RopeArgs& a, int t, int h, int cw, u32x4 w, const float4* cq,
@@ -166,29 +191,14 @@ __device__ __forceinline__ void rope_store_chunk(const RopeArgs& a, int t, int h
         const float4* csp = is_q ? cq : ck;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-#pragma clang fp contract(off)
-            // Each product and sum is rounded to fp32 on its own: no fused multiply-add.
             const float4 pair2 = csp[j >> 1];
             const float c = (j & 1) ? pair2.z : pair2.x, s = (j & 1) ? pair2.w : pair2.y;
-            const float x0 = bf16_to_f32(w[j] & 0xFFFFu), x1 = bf16_to_f32(w[j] >> 16);
-            const float r0 = x0 * c - x1 * s;
-            const float r1 = x0 * s + x1 * c;
-            w[j] = (uint32_t)f32_to_bf16_rne(r0) | ((uint32_t)f32_to_bf16_rne(r1) << 16);
+            w[j] = rotate_pair(w[j] & 0xFFFFu, w[j] >> 16, c, s);
         }
     }
-    uint16_t* dst;
-    if (is_q) {
-        dst = a.q_out + ((size_t)h * a.n_tokens + t) * D;
-    } else {
-        const int g = is_k ? h - a.n_q_heads : h - a.n_q_heads - a.n_kv_heads;
-        int64_t r = (int64_t)g * a.l_cap + a.row0 + t;
-        if (a.block_table != nullptr) {
-            r = paged_row(a.block_table, a.page_shift, a.n_kv_heads, g, a.row0 + t);
-            if (r < 0) return;  // unmapped page: nothing to write
-        }
-        dst = (is_k ? a.kc : a.vc) + (size_t)r * D;
-    }
-    *reinterpret_cast<u32x4*>(dst + 8 * cw) = w;
+    uint16_t* dst = is_q ? a.q_out + ((size_t)h * a.n_tokens + t) * D
+                         : cache_row(a, is_k, is_k ? h - a.n_q_heads : h - a.n_q_heads - a.n_kv_heads, t);
+    if (dst != nullptr) *reinterpret_cast<u32x4*>(dst + 8 * cw) = w;
 }
 
 // One work-group per token: the token's H_q + 2 H_kv head rows move in 16-byte chunks of four
@@ -213,6 +223,219 @@ __global__ __launch_bounds__(kRopeThreads) void rope_scatter_kernel(RopeArgs a) 
     }
     for (int ci = threadIdx.x; ci < n_chunks; ci += kRopeThreads)
         rope_store_chunk(a, t, ci / CPH, cw, __builtin_nontemporal_load(src + ci), cq, ck);
+}
+
+// ---- the whole stage for few tokens -------------------------------------------------------------
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kTileOut = 16;  // output rows (of W) of a tile, and the most tokens of a call
+constexpr int kFewWaves = 8;
+
+// Tokens whose normalised rows fit the LDS beside the rest (16 columns of the MFMA; more tokens go to the
+// library product).
+constexpr int few_tokens_most(int hidden) { return hidden > 4096 ? 8 : 16; }
+
+// Sum over the wave, in every lane: lane exchanges within 16 lanes, then across them.
+__device__ __forceinline__ float wave_sum(float x) {
+    auto add = [](float v, auto ctrl) {
+        return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xF, 0xF, true));
+    };
+    x = add(x, std::integral_constant<int, 0xB1>{});   // quad_perm [1, 0, 3, 2]
+    x = add(x, std::integral_constant<int, 0x4E>{});   // quad_perm [2, 3, 0, 1]
+    x = add(x, std::integral_constant<int, 0x141>{});  // row_half_mirror
+    x = add(x, std::integral_constant<int, 0x140>{});  // row_mirror
+    return pair_sum32(pair_sum16(x));
+}
+
+// RMSNorm, projection, RoPE and scatter of a few tokens in one launch.  The stage is then the weights'
+// stream (48 MiB at hidden 4096 and 6144 outputs), and the launches around a library product cost as
+// much as half of it.  One work-group per CU takes output tiles of 16 rows in turn; its waves split
+// `hidden` and run v_mfma_f32_16x16x32_bf16 (A: 16 rows of W, straight from memory; B: the normalised
+// tokens, from LDS).  Two chunks of R loads each (256 KiB per CU) are in flight from the first
+// instructions on, across tiles, behind the loads of x only, which the norm waits for; the norm and
+// the rotations are done while the first weights arrive.  The waves' partial products meet in LDS.
+// Back to back over three sets of weights, hidden 4096, 32/8 heads of 128 (a streaming read of the weights alone:
+// 8.3 us): one token 10.7 us, 4: 11.1, 16: 14.3; norm, library product and RoPE launch took 17.5.  Hidden
+// 2048, 16/8 heads: 5.2 .. 8.2 against 17.3.  Hidden 8192, 64/8 heads (24.9 us): 28.6 .. 31.9 against
+// 30.5 .. 32.6.  (Two resident 16-row work-groups per CU with their own norms instead: 14.0, 5.3 and 48.3.)
+template <int HIDDEN>
+struct FewTokensLds {
+    static constexpr int kRow = HIDDEN / 8 + 4;  // 16-byte chunks of a row, shifted by 4 per token (bank conflicts)
+    u32x4 y[few_tokens_most(HIDDEN)][kRow];      // normalised tokens
+    f32x4 part[2][kFewWaves][64];                // the waves' shares of a tile, by the tile's parity
+    float sums[kFewWaves][16];
+};
+
+// MULTI: the work-group has more than one chunk.
+template <int HIDDEN, bool MULTI>
+__device__ __forceinline__ void few_tokens_body(const FewTokensArgs& a, FewTokensLds<HIDDEN>& lds) {
+    constexpr int kThreads = kFewWaves * 64;
+    constexpr int STEPS = HIDDEN / (32 * kFewWaves);  // MFMA steps of a wave per tile
+    constexpr int R = STEPS < 16 ? STEPS : 16;        // of a chunk
+    constexpr int C = STEPS / R;                      // chunks per tile
+    constexpr int TOKENS = few_tokens_most(HIDDEN);
+    constexpr int PER = HIDDEN / 8 > kThreads ? HIDDEN / 8 / kThreads : 1;  // 16-byte chunks of a row per thread
+    static_assert(STEPS * 32 * kFewWaves == HIDDEN && C * R == STEPS, "whole steps");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, quarter = lane >> 4;
+    const int n_tokens = a.rope.n_tokens, D = a.rope.head_dim;
+    const int nq = a.rope.n_q_heads * D, nkv = a.rope.n_kv_heads * D;
+    const int n_tiles = (nq + 2 * nkv) / kTileOut;
+    const int my_tiles = (n_tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
+    const bool norm = a.gamma != nullptr;
+
+    // Where tile j of this work-group lies: matrix (Q, K, V) and first row of it.
+    auto place = [&](int j, int* row0) {
+        const int out0 = ((int)blockIdx.x + j * (int)gridDim.x) * kTileOut;
+        const int which = out0 < nq ? 0 : out0 < nq + nkv ? 1 : 2;
+        *row0 = out0 - (which == 0 ? 0 : which == 1 ? nq : nq + nkv);
+        return which;
+    };
+    // Wave j finishes tile j; its lanes rotate pairs (row0 % D + 4 quarter) / 2 and the next of token `col`.
+    int fin_row0 = 0, fin_which = 2;
+    if (wave < my_tiles) fin_which = place(wave, &fin_row0);
+    const bool rotate = a.rope.rope && fin_which < 2;
+    float theta[2] = {};
+    if (rotate) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) theta[i] = a.theta[((fin_row0 % D + 4 * quarter) >> 1) + i];
+    }
+    const u32x4* xr = reinterpret_cast<const u32x4*>(a.x);
+    const bool in_row = HIDDEN / 8 >= kThreads || tid < HIDDEN / 8;
+    u32x4 xv[TOKENS][PER], gv[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) gv[i] = norm && in_row ? reinterpret_cast<const u32x4*>(a.gamma)[i * kThreads + tid] : u32x4{};
+#pragma unroll
+    for (int t = 0; t < TOKENS; ++t)
+        if (t < n_tokens) {
+#pragma unroll
+            for (int i = 0; i < PER; ++i) xv[t][i] = in_row ? xr[t * (HIDDEN / 8) + i * kThreads + tid] : u32x4{};
+        }
+    u32x4 w[2][R];  // chunks c and c + 1 of the work-group's stream of tiles
+    const int n_chunks = my_tiles * C;
+    auto load_w = [&](u32x4 (&dst)[R], int c) __attribute__((always_inline)) {
+        int row0;
+        const int which = place(c / C, &row0);
+        const u32x4* wp = reinterpret_cast<const u32x4*>(a.w[which] + (size_t)(row0 + col) * HIDDEN +
+                                                         wave * STEPS * 32 + (c % C) * R * 32 + 8 * quarter);
+#pragma unroll
+        for (int s = 0; s < R; ++s) dst[s] = __builtin_nontemporal_load(wp + 4 * s);
+    };
+    // Loads return in order, and a wait counts the ones behind it: the weights' loads are not conditional, so
+    // that the wait for x leaves both chunks in flight, and the wait for a chunk the next one.
+    load_w(w[0], 0);
+    if constexpr (MULTI) load_w(w[1], 1);
+
+    if (norm) {
+#pragma unroll
+        for (int t = 0; t < TOKENS; ++t)
+            if (t < n_tokens) {
+                float ss = 0.f;
+#pragma unroll
+                for (int i = 0; i < PER; ++i) {
+                    ss += sum_squares(xv[t][i]);
+                    asm volatile("" : "+v"(xv[t][i]));  // (the unpacked words are not kept for the scaling: registers)
+                }
+                ss = wave_sum(ss);
+                if (lane == 0) lds.sums[wave][t] = ss;
+            }
+        __syncthreads();
+        // (every lane: the scale of token `col`, handed out below)
+        float total = 0.f;
+#pragma unroll
+        for (int i = 0; i < kFewWaves; ++i) total += lds.sums[i][col];
+        const float inv = 1.0f / sqrtf(total / (float)HIDDEN + a.eps);
+#pragma unroll
+        for (int t = 0; t < TOKENS; ++t)
+            if (t < n_tokens) {
+                const float scale = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv), t));
+#pragma unroll
+                for (int i = 0; i < PER; ++i) xv[t][i] = scale_row(xv[t][i], gv[i], scale);
+            }
+    }
+#pragma unroll
+    for (int t = 0; t < TOKENS; ++t)
+        if (t < n_tokens && in_row) {
+#pragma unroll
+            for (int i = 0; i < PER; ++i) lds.y[t][i * kThreads + tid] = xv[t][i];
+        }
+    float2 cs[2] = {};
+    if (rotate) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) cs[i] = rope_cos_sin((fin_which == 0 ? a.q_pos_base : a.kv_pos_base) + col, theta[i]);
+    }
+    __syncthreads();
+
+    const u32x4* yp = &lds.y[col < n_tokens ? col : 0][wave * STEPS * 4 + quarter];
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};  // output rows 4 quarter + i of the tile, token `col`
+    auto product = [&](const u32x4 (&wc)[R], int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < R; ++s)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wc[s]),
+                                                          __builtin_bit_cast(bf16x8_t, yp[((c % C) * R + s) * 4]), acc, 0, 0, 0);
+    };
+    auto finish = [&](int c) __attribute__((always_inline)) {  // after chunk c
+        if (c % C != C - 1) return;
+        const int j = c / C;
+        lds.part[j & 1][wave][lane] = acc;
+        acc = f32x4{0.f, 0.f, 0.f, 0.f};
+        __syncthreads();  // (the other parity's readers have passed it, so its next writers may go on)
+        if (wave != j || col >= n_tokens) return;
+        f32x4 sum = lds.part[j & 1][0][lane];
+#pragma unroll
+        for (int i = 1; i < kFewWaves; ++i) sum += lds.part[j & 1][i][lane];
+        uint32_t o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = f32_to_bf16_rne(sum[i]);
+        uint2 out;
+        out.x = rotate ? rotate_pair(o[0], o[1], cs[0].x, cs[0].y) : o[0] | (o[1] << 16);
+        out.y = rotate ? rotate_pair(o[2], o[3], cs[1].x, cs[1].y) : o[2] | (o[3] << 16);
+        const int head = fin_row0 / D;
+        uint16_t* dst = fin_which == 0 ? a.rope.q_out + ((size_t)head * n_tokens + col) * D
+                                       : cache_row(a.rope, fin_which == 1, head, col);
+        if (dst != nullptr) *reinterpret_cast<uint2*>(dst + fin_row0 % D + 4 * quarter) = out;
+    };
+    if constexpr (!MULTI) {
+        product(w[0], 0);
+        finish(0);
+    } else {
+        int c = 0;
+        for (; c + 3 < n_chunks; c += 2) {
+            product(w[0], c);
+            load_w(w[0], c + 2);
+            finish(c);
+            product(w[1], c + 1);
+            load_w(w[1], c + 3);
+            finish(c + 1);
+        }
+        if (c + 3 == n_chunks) {
+            product(w[0], c);
+            load_w(w[0], c + 2);
+            finish(c);
+            product(w[1], c + 1);
+            finish(c + 1);
+            product(w[0], c + 2);
+            finish(c + 2);
+        } else {
+            product(w[0], c);
+            finish(c);
+            product(w[1], c + 1);
+            finish(c + 1);
+        }
+    }
+}
+
+template <int HIDDEN>
+__global__ __launch_bounds__(kFewWaves * 64) void layer_few_tokens_kernel(FewTokensArgs a) {
+    __shared__ FewTokensLds<HIDDEN> lds;
+    const int n_tiles = (a.rope.n_q_heads + 2 * a.rope.n_kv_heads) * a.rope.head_dim / kTileOut;
+    constexpr bool kOneChunkTiles = HIDDEN <= 32 * kFewWaves * 16;
+    if (kOneChunkTiles && (int)(blockIdx.x + gridDim.x) >= n_tiles)
+        few_tokens_body<HIDDEN, !kOneChunkTiles>(a, lds);
+    else
+        few_tokens_body<HIDDEN, true>(a, lds);
 }
 
 }  // namespace
@@ -245,6 +468,30 @@ hipError_t launch_rope_scatter(const RopeArgs& a, const Launch& l) {
         (a.rope && a.cs == nullptr))
         return hipErrorInvalidValue;
     return launch_kernel(rope_scatter_kernel, dim3(a.n_tokens), dim3(kRopeThreads), l, a);
+}
+
+static int few_tokens_tiles(const FewTokensArgs& a) {
+    return (a.rope.n_q_heads + 2 * a.rope.n_kv_heads) * a.rope.head_dim / kTileOut;
+}
+
+bool few_tokens_supported(const FewTokensArgs& a, int n_cu) {
+    const uintptr_t align = reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.gamma) |
+                            reinterpret_cast<uintptr_t>(a.w[0]) | reinterpret_cast<uintptr_t>(a.w[1]) |
+                            reinterpret_cast<uintptr_t>(a.w[2]);
+    return a.rope.n_tokens >= 1 && a.rope.n_tokens <= few_tokens_most(a.hidden) && a.rope.head_dim % kTileOut == 0 &&
+           (align & 15) == 0 && few_tokens_tiles(a) <= kFewWaves * n_cu && (a.hidden == 1024 || a.hidden == 2048 || a.hidden == 4096 || a.hidden == 8192);
+}
+
+hipError_t launch_few_tokens(const FewTokensArgs& a, int n_cu, const Launch& l) {
+    if (!few_tokens_supported(a, n_cu)) return hipErrorInvalidValue;
+    const dim3 grid(std::min(few_tokens_tiles(a), n_cu));
+    const dim3 block(kFewWaves * 64);
+    switch (a.hidden) {
+        case 1024: return launch_kernel(layer_few_tokens_kernel<1024>, grid, block, l, a);
+        case 2048: return launch_kernel(layer_few_tokens_kernel<2048>, grid, block, l, a);
+        case 4096: return launch_kernel(layer_few_tokens_kernel<4096>, grid, block, l, a);
+        default: return launch_kernel(layer_few_tokens_kernel<8192>, grid, block, l, a);
+    }
 }
 
 }  // namespace lara

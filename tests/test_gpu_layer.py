@@ -241,3 +241,66 @@ def test_layer_at_2048_tokens_sampled_rows():
         chain, _ = orc.attention(orc.bf16_u16_to_fp32(qc), orc.bf16_u16_to_fp32(kc[:, :r0 + 64]),
                                  orc.bf16_u16_to_fp32(vc[:, :r0 + 64]), causal=True, q_pos_base=r0)
         assert float(orc.row_ulp_error(out[:, r0:r0 + 64], chain).max()) <= 3.0, r0
+
+
+@pytest.mark.parametrize("hidden,L,hq,hkv,d", [(1024, 1, 8, 2, 128), (1024, 16, 8, 2, 64), (2048, 3, 16, 8, 128),
+                                               (4096, 1, 32, 8, 128), (4096, 15, 32, 8, 128), (4096, 16, 32, 2, 64),
+                                               (4096, 17, 32, 8, 128), (8192, 1, 64, 8, 128), (8192, 8, 64, 8, 128),
+                                               (8192, 9, 8, 2, 128), (4096, 5, 1, 1, 64)])
+def test_few_tokens_stage(hidden, L, hq, hkv, d):
+    """The one-launch stage (up to 16 tokens, 8 at hidden 8192; the others take the general one): the projection
+    within its fp32 bound, RMSNorm through it, RoPE word for word, and the same words from separate weights, on
+    a paged cache and where a misaligned x sends the call to the general path (its own bound)."""
+    print(f"[layer] few tokens hidden={hidden} L={L} hq={hq} hkv={hkv} d={d}", flush=True)
+    rng = np.random.default_rng(hidden + L + d)
+    x = bf16_normal(rng, (L, hidden), 3.0)
+    wq, wk, wv = weights(rng, hq * d, hkv * d, hidden)
+    gamma = orc.fp32_to_bf16_u16((1.0 + 0.1 * rng.standard_normal(hidden)).astype(np.float32))
+    kw = dict(n_q_heads=hq, n_kv_heads=hkv, head_dim=d, max_seq_len=128)
+    with AttentionAccelerator(**kw) as acc:
+        plain = stage(acc, x, wq, wk, wv, None, rope=False, row0=3)
+        fused = stage(acc, x, wq, wk, wv, None, rope=False, row0=3, fused=True)
+        normed = stage(acc, x, wq, wk, wv, gamma, rope=False, row0=60)
+        roped = stage(acc, x, wq, wk, wv, gamma, row0=60, q_pos_base=70001, kv_pos_base=60)
+    with AttentionAccelerator(page_size=64, n_pages=3, **kw) as acc:
+        acc.reserve(0, 128)
+        paged = stage(acc, x, wq, wk, wv, gamma, row0=60, q_pos_base=70001, kv_pos_base=60)
+    y = orc.bf16_rne(lo.rms_norm_exact(x, gamma, 1e-5).astype(np.float32))
+    for got_heads, xin in ((plain, x), (normed, y)):
+        for g, w, H in zip(got_heads, (wq, wk, wv), (hq, hkv, hkv)):
+            got = orc.bf16_u16_to_fp32(g).astype(np.float64).transpose(1, 0, 2).reshape(L, H * d)
+            bound = lo.projection_error_bound(xin, w)
+            if xin is y:  # a row's y may round the other way where fp32 sums differ from float64's: one bf16 ulp of 1 % of it
+                flips = np.abs(orc.bf16_u16_to_fp32(y).astype(np.float64)) * 2.0 ** -8
+                bound = bound + 5.0 * np.sqrt(0.01 * (flips ** 2) @ (orc.bf16_u16_to_fp32(w).astype(np.float64).T ** 2))
+            err = np.abs(got - lo.project_exact(xin, w))
+            assert np.all(err <= bound), float(np.max(err / bound))
+    for a, b, c, e in zip(plain, fused, roped, paged):
+        assert np.array_equal(a, b) and np.array_equal(c, e)
+    assert np.array_equal(roped[0], lo.apply_rope(normed[0], 70001))
+    assert np.array_equal(roped[1], lo.apply_rope(normed[1], 60)) and np.array_equal(roped[2], normed[2])
+
+
+def test_few_tokens_stage_keeps_the_general_calls():
+    """What the one-launch stage does not take still runs: x off 16-byte alignment, and Q written over x."""
+    rng = np.random.default_rng(31)
+    L, hidden = 4, 1024
+    x = bf16_normal(rng, (L, hidden))
+    wq, wk, wv = weights(rng, 1024, 256, hidden)
+    gamma = orc.fp32_to_bf16_u16((1.0 + 0.1 * rng.standard_normal(hidden)).astype(np.float32))
+    with AttentionAccelerator(n_q_heads=8, n_kv_heads=2, head_dim=128, max_seq_len=64) as acc:
+        want = stage(acc, x, wq, wk, wv, gamma)
+        bufs = [dev(a) for a in (wq, wk, wv, gamma)]
+        shifted = torch.empty(L * hidden + 1, dtype=torch.int16, device="cuda")
+        shifted[1:] = dev(x).reshape(-1)
+        q = torch.empty((8, L, 128), dtype=torch.int16, device="cuda")
+        over = dev(x).clone()  # [4][1024] words: Q's [8][4][128] lands on them
+        for src, dst in ((shifted[1:], q), (over, over)):
+            print(f"[layer] general call src % 16 = {src.data_ptr() % 16} over={dst is over}", flush=True)
+            torch.cuda.synchronize()
+            acc.layer_qkv_device(src.data_ptr(), L, hidden, *(t.data_ptr() for t in bufs), dst.data_ptr())
+            torch.cuda.synchronize()
+            got = host(dst).reshape(8, L, 128)
+            diff = np.abs(orc.bf16_u16_to_fp32(got).astype(np.float64) - orc.bf16_u16_to_fp32(want[0]))
+            # the two paths sum in different orders: one bf16 ulp, and one more through the rotation
+            assert np.all(diff <= 2 * orc.bf16_ulp(np.maximum(np.abs(orc.bf16_u16_to_fp32(want[0])), 2.0 ** -6)))
