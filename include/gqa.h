@@ -80,8 +80,8 @@ extern "C" {
 #define GQA_OPT_LAYER        7 /* layered paged context: the cache layer every entry point reads and writes
                                   (0 .. n_layers-1; gqa_create_paged_layers) */
 
-/* Prefill decomposition (GQA_OPT_PREFILL_KERNEL).  SHARED: a work-group per kv head and 8 (32-row
- * block, query head) tasks shares each K/V tile over its GQA group; launches smaller than the GPU are
+/* Prefill decomposition (GQA_OPT_PREFILL_KERNEL).  SHARED: a work-group per kv head and 8 tasks of 32
+ * (query row, head) pairs shares each K/V tile over its GQA group; launches smaller than the GPU are
  * cut into KV segments merged by a second launch (GQA_OPT_PREFILL_WGS).  ROWS: a work-group per
  * (query head, 32-row block) whose waves split the keys and merge in LDS (one launch, no segments).
  * PAIRED: SHARED whose work-groups each own a long and a short causal row block (last and first),
@@ -90,8 +90,10 @@ extern "C" {
  * one KV segment; others as SHARED).
  * AUTO (default, no segment target set): PAIRED (one segment) for a causal prompt whose rows see no
  * keys before its own and whose SHARED grid holds half to one work-group per CU (a single dispatch
- * round, which longest-first dispatch cannot balance); else ROWS when the SHARED grid without
- * segments has fewer work-groups than the GPU has CUs; else SHARED -- paired when that grid is exactly
+ * round, which longest-first dispatch cannot balance); else, when the SHARED grid without segments has
+ * fewer work-groups than the GPU has CUs, ROWS or, where its estimate is the shorter (few rows after
+ * thousands of earlier keys), SHARED in one or more KV segments (several only on the first stream that
+ * needs the segments' workspace, and not under a capture); else SHARED -- paired when that grid is exactly
  * one work-group per CU (for instance a causal 2048-row chunk after earlier keys at 32q/8kv on 256
  * CUs), unpaired when larger.  gqa_last_prefill_plan reports the decomposition a launch took. */
 #define GQA_PREFILL_KERNEL_AUTO   0

@@ -20,7 +20,7 @@ namespace {
 
 constexpr int kChunkOptionQuantum = 64;  // GQA_OPT_DECODE_CHUNK: a multiple of every decode round size
 constexpr int kMinSplitCap = 256;        // the split workspace holds at least l_cap / this splits
-constexpr int kMaxPrefillSegs = 16;
+constexpr int kMaxPrefillSegs = 32;
 constexpr int32_t kMaxRows = 1 << 30;  // max_seq_len / max_q_len limit: row counts rounded up stay in int32
 constexpr double kRopeBase = 10000.0;  // theta_p = 10000^(-2p/D): hw/data/rope_theta.hex for D = 128
 constexpr int kDecodeWavesPerCu = 8;  // split planner target; one split per (sequence, kv head) once that fills the GPU
@@ -74,6 +74,8 @@ struct gqa_ctx {
     float* pre_ws = nullptr;     // prefill KV-segment partials (O, then (m, l))
     uint16_t* zero_row = nullptr;  // one zero K/V row: the prefill source of rows past kv_len
     size_t pre_ws_floats = 0;
+    bool pre_ws_bound = false;     // the stream whose automatically segmented launches use it
+    hipStream_t pre_ws_stream = nullptr;
     uint16_t* q_dev = nullptr;   // staging: max(B*H_q*D, H_q*max_q_len*D) words
     uint16_t* o_dev = nullptr;   // same size as q_dev
     float* lse_dev = nullptr;    // max(B*H_q, H_q*max_q_len)
@@ -370,6 +372,49 @@ int check_prefill_args(const gqa_ctx* c, int32_t b, int32_t q_len, int32_t q_pos
     return GQA_OK;
 }
 
+// KV segments for a launch of the shared kernel whose grid without them (`base` work-groups) is smaller
+// than the GPU, or 0 where the row-block kernel is the faster one.  The estimates are us fitted to one
+// MI355X over 5 .. 1500 rows, 0 .. 20000 earlier keys, 8/8, 16/8, 32/8 and 64/8 heads of 128 and 32/8 and 8/2 of
+// 64, most within 15 % of what was measured.  A launch's own time (back to back on one stream):
+//   row blocks: 2 + 2.5 per dispatch round, and per 256 keys 1.13 (a CU's load path) or, where the
+//     work-groups fill the GPU, 1.4 per round (the L2s' rate);
+//   shared: 4 + a 64-key block's 0.75 and 0.13 for each further task of the work-group; with segments 10 + 0.7
+//     per MB of fp32 partials (written and read) instead of 4.
+// And what it takes from launches on other streams: the larger of its time in 2.5 concurrent launches and
+// the CUs it holds (shared: the work-groups' share of the GPU times 4 + their blocks, + 0.3 per MB; with
+// segments 7.5 at least, the host's two launches).
+// Segments have to save 4 of the first (the second launch costs the host more than a stream shows) and
+// must not lose the second.  So rows stay for short histories (32/8 heads, 100 rows after 4000 keys: 25.1 us
+// against 26.5; 37 after 2000: 15.0 against 18.4) and segments win the long ones (8 after 4000: 22.3 -> 14.9;
+// 37 after 12000: 57.2 -> 28.1; 100 after 20000: 89.9 -> 49.8; 500 after 8000: 94.9 -> 74.3; 64/8, 100 after
+// 20000: 106.2 -> 77.9).
+int plan_shared_segments(int q_len, int kv_span, bool causal, int group, int n_kv_heads, int head_dim, int n_cu,
+                         int max_segs) {
+    const int base = prefill_shared_wgs(q_len, group, n_kv_heads);
+    const int tasks = prefill_tasks_per_wg(q_len, group);
+    const double per_key = head_dim > 64 ? 1.0 : 0.65;  // of the work that grows with the keys
+    const double avg_keys = causal ? kv_span - 0.5 * std::min(q_len, kv_span) : kv_span;
+    const double share = (double)((q_len + kPrefillRows - 1) / kPrefillRows) * group * n_kv_heads / n_cu;
+    const double rows_us = 2.0 + 2.5 * std::max(1.0, share) + per_key * std::max(1.13 * kv_span, 1.4 * share * avg_keys) / 256;
+    const double rows_gpu_us = std::max(0.4, 1.05 * std::min(1.0, share)) * rows_us;
+    const double block_us = per_key * (0.75 + 0.13 * (tasks - 1));
+    const int blocks = (kv_span + 63) / 64;
+    const double partial_mb = 1e-6 * q_len * group * n_kv_heads * (head_dim + 2) * 4;
+    int best = 0;
+    double best_us = rows_us;
+    for (int segs = 1; segs <= std::min(max_segs, std::max(1, n_cu / base)) && 2 * segs <= std::max(2, blocks); ++segs) {
+        const double loop_us = block_us * ((blocks + segs - 1) / segs), mb = segs > 1 ? partial_mb * segs : 0.0;
+        const double us = (segs > 1 ? 10.0 : 4.0) + 0.7 * mb + loop_us;
+        if (segs > 1 && rows_gpu_us < 7.5) break;  // the host's time for two launches
+        const double gpu_us = std::max(0.4 * us, 1.05 * ((double)(base * segs) / n_cu * (4.0 + loop_us) + 0.3 * mb));
+        if (us + (segs > 1 ? 4.0 : 0.0) < best_us && gpu_us <= rows_gpu_us) {
+            best_us = us + (segs > 1 ? 4.0 : 0.0);
+            best = segs;
+        }
+    }
+    return best;
+}
+
 int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_pos_base, int32_t kv_len,
                 int32_t kv_pos_base, int32_t causal, void* o, float* lse, hipStream_t s,
                 const void* k_new = nullptr, const void* v_new = nullptr, int32_t n_new = 0) {
@@ -419,21 +464,38 @@ int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_p
     // 23.5 vs 21.4.)  Earlier keys are read by both row blocks of a pair in step, unpaired, so
     // chunks after a history keep the row-block kernel.
     const int shared_wgs = prefill_shared_wgs(q_len, c->group, c->cfg.n_kv_heads);
+    const int paired_wgs = prefill_paired_wgs(q_len, c->cfg.n_kv_heads);
     const bool pairable = causal && c->group == 4 && q_len > kPrefillRows;
     const bool pair_auto = c->prefill_kernel == GQA_PREFILL_KERNEL_AUTO && c->prefill_wgs_opt == 0 && pairable &&
-                           kv_span <= q_len && 2 * shared_wgs >= c->n_cu && shared_wgs <= c->n_cu;
+                           kv_span <= q_len && 2 * paired_wgs >= c->n_cu && paired_wgs <= c->n_cu;
     // Launches whose shared-tile grid would not fill the GPU without KV segments take the row-block
-    // kernel (no segments, no merge launch), unless a segment target is set.
-    const bool rows = c->prefill_kernel == GQA_PREFILL_KERNEL_ROWS ||
-                      (c->prefill_kernel == GQA_PREFILL_KERNEL_AUTO && c->prefill_wgs_opt == 0 &&
-                       shared_wgs < c->n_cu && !pair_auto);
+    // kernel, or the segments that plan_shared_segments finds faster, unless a segment target is set.
+    const bool plan_auto = c->prefill_kernel == GQA_PREFILL_KERNEL_AUTO && c->prefill_wgs_opt == 0 &&
+                           shared_wgs < c->n_cu && !pair_auto;
+    auto segments = [&](int max_segs) {
+        return plan_shared_segments(q_len, kv_span, causal != 0, c->group, c->cfg.n_kv_heads, c->cfg.head_dim, c->n_cu,
+                                    max_segs);
+    };
+    int segs = plan_auto ? segments(kMaxPrefillSegs) : 0;
+    if (segs > 1) {
+        // The partials' workspace belongs to the first stream that needs it: launches on other streams and
+        // captured ones (a graph may replay beside anything) may overlap with that stream's and use none.
+        if (!c->pre_ws_bound && !stream_capturing(s)) {
+            c->pre_ws_bound = true;
+            c->pre_ws_stream = s;
+        }
+        if (!c->pre_ws_bound || c->pre_ws_stream != s || stream_capturing(s)) segs = segments(1);
+    }
     // A forced PAIRED decomposition plans one KV segment (pairs exist only in one-segment launches);
     // launches it cannot pair (not causal, group != 4, one row block) plan as SHARED.
     const bool pair_forced = c->prefill_kernel == GQA_PREFILL_KERNEL_PAIRED && pairable;
-    const int target = (pair_auto || pair_forced) ? 1 : c->prefill_wgs_opt > 0 ? c->prefill_wgs_opt : c->n_cu;
+    const int target = (pair_auto || pair_forced) ? 1 : c->prefill_wgs_opt > 0 ? c->prefill_wgs_opt
+                       : segs > 0                 ? segs * shared_wgs
+                                                  : c->n_cu;
     PrefillPlan plan = plan_prefill(q_len, kv_span, c->group, c->cfg.n_kv_heads, target, kMaxPrefillSegs);
-    if (prefill_workspace_floats(plan, q_len, c->cfg.n_q_heads, c->cfg.head_dim) > c->pre_ws_floats)
-        plan = plan_prefill(q_len, kv_span, c->group, c->cfg.n_kv_heads, 1, 1);  // one segment
+    const bool fits = prefill_workspace_floats(plan, q_len, c->cfg.n_q_heads, c->cfg.head_dim) <= c->pre_ws_floats;
+    if (!fits) plan = plan_prefill(q_len, kv_span, c->group, c->cfg.n_kv_heads, 1, 1);  // one segment
+    const bool rows = c->prefill_kernel == GQA_PREFILL_KERNEL_ROWS || (plan_auto && (segs == 0 || !fits));
     PrefillArgs a{};
     const size_t seq_off = c->paged ? 0 : (size_t)b * c->cfg.n_kv_heads * c->l_cap * c->cfg.head_dim;
     a.q = (const uint16_t*)q;
@@ -459,8 +521,8 @@ int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_p
     a.seg_len = plan.seg_len;
     a.n_segs = plan.n_segs;
     a.zero_row = c->zero_row;
-    a.part_o = reinterpret_cast<uint16_t*>(c->pre_ws);
-    a.part_ml = c->pre_ws + (size_t)plan.n_segs * c->cfg.n_q_heads * q_len * (c->cfg.head_dim / 2);
+    a.part_o = c->pre_ws;
+    a.part_ml = c->pre_ws + (size_t)plan.n_segs * c->cfg.n_q_heads * q_len * c->cfg.head_dim;
     if (rows) {
         HIP_TRY(launch_prefill_rows(c->cfg.head_dim, a, timed(c, GQA_TIMER_PREFILL, s)));
         c->last_prefill_kernel = GQA_PREFILL_KERNEL_ROWS;
@@ -471,7 +533,7 @@ int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_p
     // dispatch round (at most one work-group per CU) cannot be balanced by longest-first dispatch.
     a.pair = pairable && plan.n_segs == 1 &&
                      (c->prefill_kernel == GQA_PREFILL_KERNEL_PAIRED || pair_auto ||
-                      (c->prefill_kernel == GQA_PREFILL_KERNEL_AUTO && shared_wgs == c->n_cu))
+                      (c->prefill_kernel == GQA_PREFILL_KERNEL_AUTO && paired_wgs == c->n_cu))
                  ? 1 : 0;
     HIP_TRY(launch_prefill(c->cfg.head_dim, c->group, a, timed(c, GQA_TIMER_PREFILL, s)));
     if (plan.n_segs > 1) HIP_TRY(launch_prefill_combine(c->cfg.head_dim, a, timed(c, GQA_TIMER_COMBINE, s)));

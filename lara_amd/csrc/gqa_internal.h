@@ -129,9 +129,8 @@ struct PrefillArgs {
     float* lse;             // [H_q][q_len] or nullptr
     int32_t seg_len;        // keys per KV segment (multiple of 64)
     int32_t n_segs;         // KV segments (grid z); 1 = write the output directly
-    uint16_t* part_o;       // [n_segs][H_q][q_len][D] fp16 words: the segment's O divided by 2^e, e the
-                            //   exponent of the row's largest |O| (frexp)
-    float* part_ml;         // [n_segs][H_q][q_len][4] (running max in log2 units, sum l, e, unused)
+    float* part_o;          // [n_segs][H_q][q_len][D] fp32: the segment's un-normalised O
+    float* part_ml;         // [n_segs][H_q][q_len][2] (running max in log2 units, sum l)
     const uint16_t* zero_row;  // >= D zero words: the source of K/V rows past kv_len
     // Paged cache: block_table is sequence b's row of page indices (-1 = unmapped, read as
     // zero_row, never written), kc/vc the pools [n_pages][H_kv][2^page_shift][D]; nullptr =
@@ -220,6 +219,10 @@ hipError_t launch_prefill(int head_dim, int group, const PrefillArgs& a, const L
 hipError_t launch_prefill_rows(int head_dim, const PrefillArgs& a, const Launch& l);
 // Work-groups of launch_prefill for q_len rows without KV segments.
 int prefill_shared_wgs(int q_len, int group, int n_kv_heads);
+// Tasks of such a work-group (1 .. 8).
+int prefill_tasks_per_wg(int q_len, int group);
+// The work-groups with paired row blocks (group 4).
+int prefill_paired_wgs(int q_len, int n_kv_heads);
 // Merges the KV segments of a prefill launch with n_segs > 1.
 hipError_t launch_prefill_combine(int head_dim, const PrefillArgs& a, const Launch& l);
 

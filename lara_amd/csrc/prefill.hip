@@ -10,10 +10,11 @@
 //                                               (attn_top.sv:462-625, output_buffer.sv:226-286)
 // Like the RTL (attn_top.sv:656), P enters the PV product as bf16 while l sums the fp32 p.
 //
-// Work decomposition.  A wave owns 32 query rows of one query head; the eight waves of a
-// work-group own eight (row block, head) tasks of one KV head, heads fastest, so a GQA group
-// of 4 shares every K/V tile across its heads and two row blocks.  Keys are processed in
-// blocks of 64:
+// Work decomposition.  A wave owns a task of 32 (query row, head) pairs of one KV head, heads
+// fastest, so that few rows still fill it (9 rows of a group of 4 are two tasks, not four); the
+// eight waves of a work-group own eight consecutive tasks and share every K/V tile: a GQA group of 4
+// shares it across its heads and 64 rows.  (Paired row blocks, below, keep 32 rows of one head per
+// wave.)  Keys are processed in blocks of 64:
 //   S^T [64 keys x 32 rows] = K [64 x D] . Q^T [D x 32]   two v_mfma_f32_32x32x16_bf16 chains;
 //                                                          K from LDS (A), Q^T from VGPRs (B)
 //   O^T [D x 32 rows]      += V^T [D x 64] . P^T [64 x 32] D/32 chains of four MFMAs;
@@ -47,7 +48,6 @@ namespace {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kBN = 64;     // keys per block
 constexpr int kRows = kPrefillRows;  // query rows per wave
@@ -212,10 +212,11 @@ __device__ __forceinline__ void stash_put(uint2* stash, int col, int half, int m
     stash[2 * (col * NCH + (chunk ^ (col & (NCH - 1)))) + half] = w;
 }
 
-// Stores rows row0 .. row0 + 31 (those below q_len) of the stash to out (row r at out + r*D).  The
-// stash was written by this wave; the wait orders its LDS writes before the reads.
-template <int D>
-__device__ __forceinline__ void stash_store_rows(const uint2* stash, uint16_t* out, int row0, int q_len, int lane) {
+// Stores the stash's rows to out, [G][q_len][D]: row r of it is (row, head) pair p0 + r, heads fastest
+// (those with a row below q_len).  The stash was written by this wave; the wait orders its LDS writes
+// before the reads.
+template <int D, int G>
+__device__ __forceinline__ void stash_store_rows(const uint2* stash, uint16_t* out, int p0, int q_len, int lane) {
     constexpr int NCH = D / 8;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     const uint4* s4 = reinterpret_cast<const uint4*>(stash);
@@ -223,8 +224,9 @@ __device__ __forceinline__ void stash_store_rows(const uint2* stash, uint16_t* o
     for (int it = 0; it < D / 16; ++it) {
         const int qc = it * 64 + lane;  // chunk qc of the block: row r, chunk c
         const int r = qc / NCH, c = qc % NCH;
-        if (row0 + r < q_len)
-            *reinterpret_cast<uint4*>(out + (size_t)(row0 + r) * D + 8 * c) = s4[r * NCH + (c ^ (r & (NCH - 1)))];
+        const int row = (p0 + r) / G, head = (p0 + r) % G;
+        if (row < q_len)
+            *reinterpret_cast<uint4*>(out + ((size_t)head * q_len + row) * D + 8 * c) = s4[r * NCH + (c ^ (r & (NCH - 1)))];
     }
 }
 
@@ -268,7 +270,7 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_kernel(PrefillArgs a) {
     const int h = lin % a.n_kv_heads;                    // kv head
     const int wx = lin / a.n_kv_heads;                   // task group of the head
     const int n_rb = (a.q_len + kRows - 1) / kRows;
-    const int n_tasks = n_rb * G;
+    const int n_tasks = PAIR ? n_rb * G : (a.q_len * G + kRows - 1) / kRows;
     // Causal row blocks grow in work with their index: the largest go to the work-groups the
     // dispatcher starts first (longest first), so a grid larger than the GPU balances.
     // PAIR (a causal grid of one dispatch round): work-group p owns row blocks L = n_rb - 1 - p and
@@ -278,19 +280,19 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_kernel(PrefillArgs a) {
     // work-group then carries about (keys(L) + keys(S)) / 2 keys per wave, instead of keys(L) for
     // the work-groups of the last row blocks.
     const int wg_x = (a.causal && !PAIR) ? (int)(gridDim.x - 1 - wx) : wx;
-    const int task = PAIR ? (n_rb - 1 - wx) * G + (wave & 3) : wg_x * kWaves + wave;
-    const bool active = task < n_tasks;
-    const int g = task % G;
+    // The tasks are dealt evenly (9 of them as 5 and 4): a work-group's time grows with its tasks.
+    const int wg_tasks = (n_tasks + (int)gridDim.x - 1) / (int)gridDim.x;
+    const int task = PAIR ? (n_rb - 1 - wx) * G + (wave & 3) : wg_x * wg_tasks + wave;
+    const bool active = task < n_tasks && (PAIR || wave < wg_tasks);
     const int rb = task / G;  // PAIR: row block L (every wave's last)
-    const int hq = h * G + g;
     const bool has_s = PAIR && wx < rb;                 // PAIR: the work-group has a row block S
     const int rb_first = (has_s && wave >= 4) ? wx : rb;  // the row block the wave starts on
 
-    // Keys a row block needs: [0, kv_limit) (causal rows stop at their diagonal).
-    auto kv_limit = [&](int row_block) {
+    // Keys a row block (PAIR) or a task needs: [0, kv_limit) (causal rows stop at their diagonal).
+    auto kv_limit = [&](int unit) {
         int hi = a.kv_len;
         if (a.causal) {
-            const int last_row = min(a.q_len, (row_block + 1) * kRows) - 1;
+            const int last_row = min(a.q_len, PAIR ? (unit + 1) * kRows : ((unit + 1) * kRows - 1) / G + 1) - 1;
             hi = min(hi, a.q_pos_base + last_row - a.kv_pos_base + 1);
         }
         return max(hi, 0);
@@ -323,9 +325,9 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_kernel(PrefillArgs a) {
             }
         }
     };
-    const int last_task = min(n_tasks, (wg_x + 1) * kWaves) - 1;
-    const int wg_hi = PAIR ? kv_limit(rb) : kv_limit(last_task / G);  // row blocks grow with the task index
-    int wave_hi = active ? kv_limit(rb_first) : 0;
+    const int last_task = min(n_tasks, (wg_x + 1) * wg_tasks) - 1;
+    const int wg_hi = kv_limit(PAIR ? rb : last_task);  // the keys grow with the task index
+    int wave_hi = active ? kv_limit(PAIR ? rb_first : task) : 0;
     const int seg_begin = blockIdx.z * a.seg_len;
     // With several segments, one that no row of this work-group reaches is not read by the
     // merge; a single segment always reaches the epilogue (rows without keys output 0).
@@ -339,7 +341,10 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_kernel(PrefillArgs a) {
     const int col = lane & 31;   // query row within the wave's block (MFMA column)
     const int half = lane >> 5;  // which 8 k-values of a step this lane carries
     int cur_rb = rb_first;       // the row block the wave works on (PAIR: S, then L)
-    const int row0 = cur_rb * kRows + col;
+    // The lane's query row and head: row `col` of its row block (PAIR), or pair task * 32 + col of the kv
+    // head's (row, head) pairs, heads fastest.
+    const int row0 = PAIR ? cur_rb * kRows + col : (task * kRows + col) / G;
+    const int hq = h * G + (PAIR ? task : task * kRows + col) % G;
     const bool row0_ok = active && row0 < a.q_len;
     const int q_pos0 = a.q_pos_base + row0;
 
@@ -521,9 +526,9 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_kernel(PrefillArgs a) {
         const int row = PAIR ? cur_rb * kRows + col : row0;
         const bool row_ok = PAIR ? active && row < a.q_len : row0_ok;
         const int q_pos = PAIR ? a.q_pos_base + row : q_pos0;
-        const int rb_now = PAIR ? cur_rb : rb;
+        const int first_row = PAIR ? cur_rb * kRows : task * kRows / G;
         const bool need_mask = (jb + 32 * NT > a.kv_len) ||
-                               (a.causal && a.kv_pos_base + jb + 32 * NT - 1 > a.q_pos_base + rb_now * kRows);
+                               (a.causal && a.kv_pos_base + jb + 32 * NT - 1 > a.q_pos_base + first_row);
         if (need_mask) {
 #pragma unroll
             for (int kt = 0; kt < NT; ++kt)
@@ -722,7 +727,7 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_kernel(PrefillArgs a) {
         }
     }
 
-    const int row = rb * kRows + col;  // the wave's last row block (PAIR: L)
+    const int row = PAIR ? rb * kRows + col : row0;  // (PAIR: of the wave's last row block, L)
     const bool row_ok = active && row < a.q_len;
     if constexpr (PAIR) {
         const int q4 = wave & 3;
@@ -771,12 +776,12 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_kernel(PrefillArgs a) {
                     w.y = (uint32_t)f32_to_bf16_rne(v2) | ((uint32_t)f32_to_bf16_rne(v3) << 16);
                     stash_put<D>(stash, col, half, mt, r4, w);
                 }
-            stash_store_rows<D>(stash, a.out + (size_t)hq * a.q_len * D, rb * kRows, a.q_len, lane);
+            stash_store_rows<D, 1>(stash, a.out + (size_t)hq * a.q_len * D, rb * kRows, a.q_len, lane);
             if (row_ok && half == 0 && a.lse != nullptr)
                 a.lse[(size_t)hq * a.q_len + row] = l_sum > 0.f ? (M + log2f(l_sum)) * kLn2 : -INFINITY;
         } else if (has_s) {
             // S's output rows from the stash leave_s filled.
-            stash_store_rows<D>(reinterpret_cast<const uint2*>(&lds_q[q4][0][0]), a.out + (size_t)hq * a.q_len * D,
+            stash_store_rows<D, 1>(reinterpret_cast<const uint2*>(&lds_q[q4][0][0]), a.out + (size_t)hq * a.q_len * D,
                                 wx * kRows, a.q_len, lane);
             const int srow = wx * kRows + col;
             if (half == 0 && a.lse != nullptr && srow < a.q_len) a.lse[(size_t)hq * a.q_len + srow] = lse_s;
@@ -789,30 +794,16 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_kernel(PrefillArgs a) {
         if (!row_ok) return;
         // Rows this wave never reached in the segment are not read by the merge.
         if (seg_begin >= wave_hi) return;
-        // The segment's unnormalised O in fp16, divided by the power of two 2^e just above the row's
-        // largest |O| (exact, any magnitude) so every dim keeps 11 significant bits relative to the
-        // row (a bf16 ulp is 8), and (m, l, e) in fp32: half the bytes of an fp32 partial, written
-        // here and read once by the merge.
+        // The segment's unnormalised O and (m, l), fp32, written here and read once by the merge.
         const size_t prow = ((size_t)blockIdx.z * a.n_q_heads + hq) * a.q_len + row;
-        float amax = 0.f;
+        float* po = a.part_o + prow * D;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(o[mt][i]));
-        amax = fmaxf(amax, half_swap(amax, half));  // the row's other half-wave
-        int e = 0;
-        if (amax > 0.f) (void)frexpf(amax, &e);  // amax in [2^(e-1), 2^e)
-        uint16_t* po = a.part_o + prow * D;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                const f16x4 w = {(_Float16)ldexpf(o[mt][4 * r4 + 0], -e), (_Float16)ldexpf(o[mt][4 * r4 + 1], -e),
-                                 (_Float16)ldexpf(o[mt][4 * r4 + 2], -e), (_Float16)ldexpf(o[mt][4 * r4 + 3], -e)};
-                *reinterpret_cast<uint2*>(po + mt * 32 + 8 * r4 + 4 * half) = __builtin_bit_cast(uint2, w);
-            }
-        if (half == 0)
-            *reinterpret_cast<float4*>(a.part_ml + prow * 4) = make_float4(m_run, l_row, (float)e, 0.f);
+            for (int r4 = 0; r4 < 4; ++r4)
+                *reinterpret_cast<float4*>(po + mt * 32 + 8 * r4 + 4 * half) =
+                    make_float4(o[mt][4 * r4 + 0], o[mt][4 * r4 + 1], o[mt][4 * r4 + 2], o[mt][4 * r4 + 3]);
+        if (half == 0) *reinterpret_cast<float2*>(a.part_ml + prow * 2) = make_float2(m_run, l_row);
         return;
     }
     // The rows are staged in the two ring stages no wave reads any more: block b sits in stage b % NST
@@ -832,7 +823,7 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_kernel(PrefillArgs a) {
             w.y = (uint32_t)f32_to_bf16_rne(o[mt][4 * r4 + 2] * inv) | ((uint32_t)f32_to_bf16_rne(o[mt][4 * r4 + 3] * inv) << 16);
             stash_put<D>(stash, col, half, mt, r4, w);
         }
-    stash_store_rows<D>(stash, a.out + (size_t)hq * a.q_len * D, rb * kRows, a.q_len, lane);
+    stash_store_rows<D, G>(stash, a.out + (size_t)h * G * a.q_len * D, task * kRows, a.q_len, lane);
     if (row_ok && half == 0 && a.lse != nullptr)
         a.lse[(size_t)hq * a.q_len + row] = l_row > 0.f ? (m_run + log2f(l_row)) * kLn2 : -INFINITY;
 }
@@ -1261,12 +1252,10 @@ hipError_t launch_prefill_rows_t(const PrefillArgs& a, const Launch& l) {
 // Merge of a row's KV segments.  Segment s holds keys [s*seg_len, (s+1)*seg_len); a row
 // reads the segments below its own key limit, which are exactly the ones prefill_kernel
 // wrote for it.  A work-group merges kMergeRows rows of one query head; each row is handled
-// by D/8 threads owning eight dims (16-byte fp16 loads).  The (m, l, scale) rows and O slices
-// of up to kMergeBatch segments are loaded together, so a row pays one memory latency per batch.
+// by D/8 threads owning eight dims.  The (m, l) and O slices of kMergeBatch segments are loaded
+// together, so a row pays one memory latency per batch.
 constexpr int kMergeRows = 16;
 constexpr int kMergeBatch = 8;
-constexpr int kMaxMergeSegs = 16;  // segments a launch may have (the host planner's cap)
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 template <int D>
 __global__ __launch_bounds__(kMergeRows * D / 8) void prefill_combine_kernel(PrefillArgs a) {
@@ -1281,71 +1270,59 @@ __global__ __launch_bounds__(kMergeRows * D / 8) void prefill_combine_kernel(Pre
     const int n_valid = min(a.n_segs, (hi + a.seg_len - 1) / a.seg_len);
     const size_t seg_stride = (size_t)a.n_q_heads * a.q_len;
     const size_t prow = (size_t)hq * a.q_len + row;
-    const float4* ml = reinterpret_cast<const float4*>(a.part_ml) + prow;
-    const uint4* po = reinterpret_cast<const uint4*>(a.part_o) + prow * TPR + d8;
-    // Segment s contributes 2^(m_s - M) * v_s * 2^(e_s) (M the largest m).  Split its log2 weight
-    // into an integer n_s and a fraction: the contribution's exponent is x_s = e_s + n_s, and O
-    // accumulates relative to X = max_s x_s, so the dominant contributions are scaled by about one
-    // and every term is scaled down by an exact power of two: nothing overflows, and nothing that
-    // matters to the sum is flushed, whatever the partials' magnitudes.
-    float4 e[kMaxMergeSegs];  // (m, l, exponent, -) of each segment
+    const float2* ml = reinterpret_cast<const float2*>(a.part_ml) + prow;
+    const float4* po = reinterpret_cast<const float4*>(a.part_o) + (prow * TPR + d8) * 2;
+    float M = -INFINITY, L = 0.f;
+    float O[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int j0 = 0; j0 < n_valid; j0 += kMergeBatch) {
+        float2 e[kMergeBatch];
+        float4 v[kMergeBatch][2];
 #pragma unroll
-    for (int j = 0; j < kMaxMergeSegs; ++j)
-        e[j] = j < n_valid ? ml[(size_t)j * seg_stride] : make_float4(-INFINITY, 0.f, 0.f, 0.f);
-    float M = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < kMaxMergeSegs; ++j) M = fmaxf(M, e[j].x);
-    uint4 w = {0u, 0u, 0u, 0u};
-    float Ls = 0.f;
-    if (M != -INFINITY) {
-        int n[kMaxMergeSegs];
-        int X = INT_MIN;
-#pragma unroll
-        for (int j = 0; j < kMaxMergeSegs; ++j) {
-            n[j] = (int)fmaxf(floorf(e[j].x - M), -1024.f);  // -1024 for an empty segment (m = -inf)
-            if (e[j].x != -INFINITY) X = max(X, (int)e[j].z + n[j]);
-            Ls = fmaf(__builtin_amdgcn_exp2f(e[j].x - M), e[j].y, Ls);
+        for (int j = 0; j < kMergeBatch; ++j) {
+            const size_t at = (size_t)min(j0 + j, n_valid - 1) * seg_stride;
+            e[j] = ml[at];
+            v[j][0] = po[at * TPR * 2];
+            v[j][1] = po[at * TPR * 2 + 1];
         }
-        float O[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        float m = M;
 #pragma unroll
-        for (int j0 = 0; j0 < kMaxMergeSegs; j0 += kMergeBatch) {
-            if (j0 >= n_valid) break;
-            f16x8 v[kMergeBatch];
+        for (int j = 0; j < kMergeBatch; ++j) m = fmaxf(m, e[j].x);
+        const float keep = M == m ? 1.f : __builtin_amdgcn_exp2f(M - m);
+        M = m;
+        L *= keep;
 #pragma unroll
-            for (int j = 0; j < kMergeBatch; ++j)
-                v[j] = j0 + j < n_valid ? __builtin_bit_cast(f16x8, po[(size_t)(j0 + j) * seg_stride * TPR])
-                                        : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        for (int i = 0; i < 8; ++i) O[i] *= keep;
 #pragma unroll
-            for (int j = 0; j < kMergeBatch; ++j) {
-                const float4& ej = e[j0 + j];
-                const float wo = ej.x == -INFINITY ? 0.f
-                                                   : ldexpf(__builtin_amdgcn_exp2f(ej.x - M - (float)n[j0 + j]),
-                                                            (int)ej.z + n[j0 + j] - X);
+        for (int j = 0; j < kMergeBatch; ++j) {
+            const float w = j0 + j < n_valid && e[j].x != -INFINITY ? __builtin_amdgcn_exp2f(e[j].x - m) : 0.f;
+            L = fmaf(w, e[j].y, L);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) O[i] = fmaf(wo, (float)v[j][i], O[i]);
+            for (int i = 0; i < 4; ++i) {
+                O[i] = fmaf(w, reinterpret_cast<const float*>(&v[j][0])[i], O[i]);
+                O[4 + i] = fmaf(w, reinterpret_cast<const float*>(&v[j][1])[i], O[4 + i]);
             }
         }
-        // out = O * 2^X / Ls, scaled back in one exact step after the division.
-        const float inv = Ls > 0.f ? 1.f / Ls : 0.f;
-        float r8[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) r8[i] = ldexpf(O[i] * inv, X);
-        w.x = (uint32_t)f32_to_bf16_rne(r8[0]) | ((uint32_t)f32_to_bf16_rne(r8[1]) << 16);
-        w.y = (uint32_t)f32_to_bf16_rne(r8[2]) | ((uint32_t)f32_to_bf16_rne(r8[3]) << 16);
-        w.z = (uint32_t)f32_to_bf16_rne(r8[4]) | ((uint32_t)f32_to_bf16_rne(r8[5]) << 16);
-        w.w = (uint32_t)f32_to_bf16_rne(r8[6]) | ((uint32_t)f32_to_bf16_rne(r8[7]) << 16);
     }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    uint4 w;
+    w.x = (uint32_t)f32_to_bf16_rne(O[0] * inv) | ((uint32_t)f32_to_bf16_rne(O[1] * inv) << 16);
+    w.y = (uint32_t)f32_to_bf16_rne(O[2] * inv) | ((uint32_t)f32_to_bf16_rne(O[3] * inv) << 16);
+    w.z = (uint32_t)f32_to_bf16_rne(O[4] * inv) | ((uint32_t)f32_to_bf16_rne(O[5] * inv) << 16);
+    w.w = (uint32_t)f32_to_bf16_rne(O[6] * inv) | ((uint32_t)f32_to_bf16_rne(O[7] * inv) << 16);
     *reinterpret_cast<uint4*>(a.out + prow * D + 8 * d8) = w;
-    if (d8 == 0 && a.lse != nullptr) a.lse[prow] = Ls > 0.f ? (M + log2f(Ls)) * kLn2 : -INFINITY;
+    if (d8 == 0 && a.lse != nullptr) a.lse[prow] = L > 0.f ? (M + log2f(L)) * kLn2 : -INFINITY;
 }
+
+// Tasks of a kv head: 32 (query row, head) pairs each.
+int prefill_tasks(int q_len, int group) { return (int)(((int64_t)q_len * group + kRows - 1) / kRows); }
 
 template <int D, int G>
 hipError_t launch_prefill_t(const PrefillArgs& a, const Launch& l) {
-    const int n_rb = (a.q_len + kRows - 1) / kRows;
-    const int n_tasks = n_rb * G;
+    const int n_tasks = prefill_tasks(a.q_len, G);
     dim3 grid((n_tasks + kWaves - 1) / kWaves, a.n_kv_heads, a.n_segs);
     if constexpr (G == 4) {
         if (a.pair) {
+            grid.x = ((a.q_len + kRows - 1) / kRows + 1) / 2;
             // Paired row blocks: causal, one segment (the whole key range in one launch).
             if (!a.causal || a.n_segs != 1) return hipErrorInvalidValue;
             if (a.block_table != nullptr)
@@ -1362,8 +1339,7 @@ hipError_t launch_prefill_t(const PrefillArgs& a, const Launch& l) {
 constexpr int kMinSegBlocks = 2;  // key blocks per KV segment, at least
 
 PrefillPlan plan_prefill(int q_len, int kv_span, int group, int n_kv_heads, int target_wgs, int max_segs) {
-    const int n_rb = (q_len + kRows - 1) / kRows;
-    const int base = ((n_rb * group + kWaves - 1) / kWaves) * n_kv_heads;
+    const int base = prefill_shared_wgs(q_len, group, n_kv_heads);
     const int blocks = (kv_span + kBN - 1) / kBN;
     int segs = (target_wgs + base - 1) / base;
     segs = min(segs, max_segs);
@@ -1376,11 +1352,10 @@ PrefillPlan plan_prefill(int q_len, int kv_span, int group, int n_kv_heads, int 
 
 size_t prefill_workspace_floats(const PrefillPlan& p, int q_len, int n_q_heads, int head_dim) {
     if (p.n_segs <= 1) return 0;
-    return (size_t)p.n_segs * n_q_heads * q_len * (head_dim / 2 + 4);  // fp16 O row + (m, l, scale, -)
+    return (size_t)p.n_segs * n_q_heads * q_len * (head_dim + 2);  // O row + (m, l)
 }
 
 hipError_t launch_prefill_combine(int head_dim, const PrefillArgs& a, const Launch& l) {
-    if (a.n_segs > kMaxMergeSegs) return hipErrorInvalidValue;
     const dim3 grid((a.q_len + kMergeRows - 1) / kMergeRows, a.n_q_heads);
     if (head_dim == 128) return launch_kernel(prefill_combine_kernel<128>, grid, dim3(kMergeRows * 16), l, a);
     if (head_dim == 64) return launch_kernel(prefill_combine_kernel<64>, grid, dim3(kMergeRows * 8), l, a);
@@ -1395,8 +1370,15 @@ hipError_t launch_prefill_rows(int head_dim, const PrefillArgs& a, const Launch&
 }
 
 int prefill_shared_wgs(int q_len, int group, int n_kv_heads) {
-    return ((q_len + kRows - 1) / kRows * group + kWaves - 1) / kWaves * n_kv_heads;
+    return (prefill_tasks(q_len, group) + kWaves - 1) / kWaves * n_kv_heads;
 }
+
+int prefill_tasks_per_wg(int q_len, int group) {
+    const int tasks = prefill_tasks(q_len, group), wgs = (tasks + kWaves - 1) / kWaves;
+    return (tasks + wgs - 1) / wgs;
+}
+
+int prefill_paired_wgs(int q_len, int n_kv_heads) { return ((q_len + kRows - 1) / kRows + 1) / 2 * n_kv_heads; }
 
 bool prefill_supported(int head_dim, int group) {
     return (head_dim == 64 || head_dim == 128) && (group == 1 || group == 2 || group == 4 || group == 8 || group == 16);

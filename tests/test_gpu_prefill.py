@@ -460,3 +460,80 @@ def test_prefill_cancelling_v_rows_within_the_weight_rounding_bound(kernel):
     assert float(err.max()) <= 1.0
     rel = np.abs(np.expm1(lse.astype(np.float64) - ref_lse))
     assert float(rel.max()) <= L_RTOL
+
+
+@pytest.mark.parametrize("hq,hkv,d,q_len,history,causal,paged,segments", [
+    (32, 8, 128, 1, 8000, True, False, True), (32, 8, 128, 9, 8000, True, True, True),
+    (32, 8, 128, 37, 7000, True, False, True), (32, 8, 128, 37, 7013, False, True, True),
+    (8, 8, 128, 33, 6000, True, False, True), (16, 8, 128, 40, 9000, True, False, True),
+    (32, 2, 64, 7, 9000, True, False, True), (64, 8, 128, 20, 9000, True, True, True),
+    (32, 8, 128, 700, 300, True, False, False), (64, 8, 128, 600, 1500, True, False, False),
+    (32, 8, 128, 37, 500, True, False, False)])
+def test_few_rows_after_a_long_history_take_segments(hq, hkv, d, q_len, history, causal, paged, segments):
+    """AUTO for few rows after thousands of keys: shared tiles in several KV segments (32 (row, head) pairs a
+    task, heads fastest, fp32 partials), one segment or row blocks where those are estimated shorter; with the
+    rows' own append, against the oracle."""
+    rng = np.random.default_rng(5000 + q_len + history + d)
+    kv_len = history + q_len
+    print(f"[segments] hq={hq} hkv={hkv} d={d} q_len={q_len} history={history} paged={paged}", flush=True)
+    q = bf16_normal(rng, (hq, q_len, d))
+    k = bf16_normal(rng, (hkv, kv_len, d))
+    v = bf16_normal(rng, (hkv, kv_len, d))
+    extra = dict(page_size=64, n_pages=-(-kv_len // 64)) if paged else {}
+    with AttentionAccelerator(n_q_heads=hq, n_kv_heads=hkv, head_dim=d, max_seq_len=kv_len, max_q_len=max(q_len, 64),
+                              **extra) as acc:
+        if paged:
+            acc.reserve(0, kv_len)
+        acc.load_kv(k[:, :history], v[:, :history])
+        out, lse = acc.prefill_chunk(q, q_pos_base=history, kv_len=kv_len, causal=causal, k_rows=k[:, history:],
+                                     v_rows=v[:, history:], return_lse=True)
+        kernel, segs = acc.last_prefill_plan()
+        assert (segs > 1) == segments and (kernel == "shared" or not segments)
+        kr, vr = acc.read_kv(0, 0, kv_len)
+    assert np.array_equal(kr, k) and np.array_equal(vr, v)
+    ref, ref_lse = oracle_for(q, k, v, causal=causal, q_pos_base=history)
+    check_rows(out, lse, ref, ref_lse)
+
+
+def test_segment_workspace_stays_with_its_stream():
+    """Automatic segments only on the first stream that needed them: another stream's launch and a captured one
+    share no workspace with it (row blocks), and every result holds with the three in flight together."""
+    torch = pytest.importorskip("torch")
+    import ctypes
+
+    from lara_amd import _lib
+
+    rng = np.random.default_rng(5100)
+    hq, hkv, d, q_len, kv_len = 32, 8, 128, 16, 9000
+    k, v = bf16_normal(rng, (hkv, kv_len, d)), bf16_normal(rng, (hkv, kv_len, d))
+    qs = [bf16_normal(rng, (hq, q_len, d)) for _ in range(3)]
+    with AttentionAccelerator(max_seq_len=kv_len, max_q_len=64) as acc:
+        acc.load_kv(k, v)
+        q_dev = [torch.from_numpy(q.view(np.int16)).cuda() for q in qs]
+        o_dev = [torch.zeros_like(q) for q in q_dev]
+        torch.cuda.synchronize()
+
+        def launch(i, stream):
+            _lib.check(acc._lib.gqa_prefill_device(acc._ctx, 0, ctypes.c_void_p(q_dev[i].data_ptr()), q_len,
+                                                   kv_len - q_len, kv_len, 0, 1, ctypes.c_void_p(o_dev[i].data_ptr()),
+                                                   None, ctypes.c_void_p(stream)), "prefill")
+            return acc.last_prefill_plan()
+
+        s0, s1 = torch.cuda.Stream(), torch.cuda.Stream()
+        assert launch(0, s0.cuda_stream)[1] > 1
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s0):
+            assert launch(2, s0.cuda_stream) == ("rows", 1)
+        for _ in range(3):
+            for o in o_dev:
+                o.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(s1):
+                graph.replay()
+            assert launch(0, s0.cuda_stream)[1] > 1
+            assert launch(1, s1.cuda_stream) == ("rows", 1)
+            torch.cuda.synchronize()
+            for q, o in zip(qs, o_dev):
+                ref, _ = oracle_for(q, k, v, causal=True, q_pos_base=kv_len - q_len)
+                check_rows(o.cpu().numpy().view(np.uint16), None, ref, None)
