@@ -761,6 +761,27 @@ class AttentionAccelerator:
                        _lib.as_u16_ptr(out), lse_ptr)
         return (out, lse) if return_lse else out
 
+    def _finish_transaction(self, prof: RunProfile, L: int, timeout_ms: int | None):
+        """Wait for the started transaction and copy its output: (words, perf counters).  Without a timeout the
+        read-back starts at once and takes the output as it arrives; the wait is then the time before the device's
+        own output copy (its share of the read-back is ``output_dma_transfer_ms`` either way)."""
+        t = time.perf_counter()
+        if timeout_ms is not None:
+            self.wait_done(None, None, None, L, timeout_ms=timeout_ms)
+            prof.request_service_ms = (time.perf_counter() - t) * 1000.0
+            t = time.perf_counter()
+        words = self.readback_o(L)
+        elapsed_ms = (time.perf_counter() - t) * 1000.0
+        if timeout_ms is None:
+            self.wait_done(None, None, None, L)  # error status, if any, as wait_done reports it
+        perf = self.read_perf()
+        if timeout_ms is None:
+            copy_ms = perf["stall_cycles"] / (self._pl_clock_mhz * 1000.0) if self._pl_clock_mhz > 0 else 0.0
+            prof.request_service_ms = max(elapsed_ms - copy_ms, 0.0)
+            elapsed_ms -= prof.request_service_ms
+        prof.output_dma_transfer_ms = elapsed_ms
+        return words, perf
+
     def run_attention(
         self,
         q_heads: np.ndarray,
@@ -826,14 +847,7 @@ class AttentionAccelerator:
         prof.output_dma_bytes = o_bytes
 
         self.start()
-        t = time.perf_counter()
-        self.wait_done(q_u16, k_u16, v_u16, L, timeout_ms=timeout_ms)
-        prof.request_service_ms = (time.perf_counter() - t) * 1000.0
-
-        t = time.perf_counter()
-        result = self.readback_o(L)
-        prof.output_dma_transfer_ms = (time.perf_counter() - t) * 1000.0
-        perf = self.read_perf()
+        result, perf = self._finish_transaction(prof, L, timeout_ms)
         prof.clock_mhz = self._pl_clock_mhz
         prof.pl_total_cycles = perf["cycles"]
         prof.pl_mac_cycles = perf["mac_cycles"]
@@ -926,13 +940,7 @@ class AttentionAccelerator:
 
         attention_start = time.perf_counter()
         self.start()
-        t = time.perf_counter()
-        self.wait_done(None, None, None, L, timeout_ms=timeout_ms)
-        prof.request_service_ms = (time.perf_counter() - t) * 1000.0
-        t = time.perf_counter()
-        words = self.readback_o(L)
-        prof.output_dma_transfer_ms = (time.perf_counter() - t) * 1000.0
-        perf = self.read_perf()
+        words, perf = self._finish_transaction(prof, L, timeout_ms)
         prof.clock_mhz = self._pl_clock_mhz
         prof.pl_total_cycles = perf["cycles"]
         prof.pl_mac_cycles = perf["mac_cycles"]

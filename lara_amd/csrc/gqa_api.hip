@@ -40,6 +40,9 @@ struct Txn {
 // n_tokens), bf16 in and out, fp32 accumulation: the hipBLASLt descriptors, the candidates its
 // heuristic ranks first (workspace up to kProjectionWorkspace bytes) and the one in use: the
 // heuristic's first until the first call outside a graph capture has timed them all.
+constexpr int kOutputParts = 4;              // a large transaction's output comes back in this many copies
+constexpr size_t kOutputPartBytes = 256 << 10;  // of at least this size
+constexpr size_t kKvStageBytes = 8u << 20;
 constexpr int kProjectionCandidates = 8;
 constexpr size_t kProjectionWorkspace = 32u << 20;
 struct ProjectionPlan {
@@ -84,6 +87,9 @@ struct gqa_ctx {
     uint16_t* rows_dev = nullptr;  // [2][B][H_kv][D] append staging
     uint16_t* new_dev = nullptr;   // [2][H_kv][max_q_len][D] chunk-append staging
     uint16_t* o_pinned = nullptr;  // transaction output (host, pinned)
+    bool q_in_flight = false;      // it may still be the source of a submitted Q's copy
+    uint8_t* kv_pinned = nullptr;  // staging of gqa_load_kv (host, pinned; idle between calls)
+    size_t kv_pinned_bytes = 0;
     size_t stage_words = 0;
     size_t lse_words = 0;
     int chunk_opt = 0;
@@ -95,6 +101,7 @@ struct gqa_ctx {
     hipEvent_t* ev_pool[GQA_TIMER_COUNT] = {};
     int ev_count[GQA_TIMER_COUNT] = {};
     hipEvent_t ev_t[4] = {};     // transaction: copy-in start, kernel start, kernel end, done
+    hipEvent_t ev_part[kOutputParts - 1] = {};  // its output's parts but the last have arrived
     float last_us = 0.f;
     double clock_mhz = 0.0;
     int n_cu = 256;  // compute units of the device (the planners' work-group targets scale with it)
@@ -551,6 +558,33 @@ int finish_sync(gqa_ctx* c) {
     return GQA_OK;
 }
 
+// The copies a transaction's Q goes and its output comes back in: one is staged, or handed on by
+// gqa_read_output, while the other way's DMA moves the next.
+int output_parts(size_t bytes) { return (int)std::max<size_t>(1, std::min<size_t>(kOutputParts, bytes / kOutputPartBytes)); }
+size_t output_part(size_t bytes, int parts, int i) { return i == parts ? bytes : bytes / parts / 64 * 64 * i; }
+
+// Waits for ev: spinning for kSpinUs, about the longest transaction of the board's size (a sleep takes 70 us
+// at the least and would be most of a short one), then between naps.  timeout_ms < 0 waits for ever.
+constexpr double kSpinUs = 1000.0;
+int wait_event(hipEvent_t ev, int32_t timeout_ms) {
+    struct timespec t0, t1;
+    clock_gettime(CLOCK_MONOTONIC, &t0);
+    for (;;) {
+        const hipError_t e = hipEventQuery(ev);
+        if (e == hipSuccess) return GQA_OK;
+        if (e != hipErrorNotReady) {
+            last_hip_error(e, "hipEventQuery");
+            return GQA_ERR_HIP;
+        }
+        clock_gettime(CLOCK_MONOTONIC, &t1);
+        const double us = (t1.tv_sec - t0.tv_sec) * 1e6 + (t1.tv_nsec - t0.tv_nsec) * 1e-3;
+        if (timeout_ms >= 0 && us > timeout_ms * 1e3) return GQA_ERR_TIMEOUT;
+        if (us < kSpinUs) continue;
+        struct timespec nap = {0, 20000};
+        nanosleep(&nap, nullptr);
+    }
+}
+
 int txn_idle(gqa_ctx* c) {
     // A transaction in flight blocks every other use of the context's staging buffers.
     if (!c->txn.running) return GQA_OK;
@@ -943,6 +977,7 @@ int create_ctx(const gqa_config* cfg, int32_t page_size, int32_t n_pages, int32_
     if (rc == GQA_OK) {
         bool ok = hipEventCreate(&c->ev_begin) == hipSuccess && hipEventCreate(&c->ev_end) == hipSuccess;
         for (int i = 0; i < 4 && ok; ++i) ok = hipEventCreate(&c->ev_t[i]) == hipSuccess;
+        for (hipEvent_t& e : c->ev_part) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
         if (!ok) rc = GQA_ERR_HIP;
     }
     // Zero the caches (every layer's pool) once so rows beyond every sequence's length hold finite words.
@@ -1130,6 +1165,9 @@ int gqa_destroy(gqa_ctx* c) {
     (void)hipFree(c->new_dev);
     (void)hipFree(c->table_dev);
     if (c->o_pinned) (void)hipHostFree(c->o_pinned);
+    if (c->kv_pinned) (void)hipHostFree(c->kv_pinned);
+    for (hipEvent_t e : c->ev_part)
+        if (e) (void)hipEventDestroy(e);
     if (c->ev_begin) (void)hipEventDestroy(c->ev_begin);
     if (c->ev_end) (void)hipEventDestroy(c->ev_end);
     for (int i = 0; i < GQA_TIMER_COUNT; ++i) {
@@ -1325,6 +1363,36 @@ int gqa_load_kv(gqa_ctx* c, int32_t b, int32_t start_pos, int32_t n, const uint1
     }
     const size_t D = c->cfg.head_dim;
     const size_t row_bytes = D * 2;
+    // Up to kKvStageBytes go through pinned memory, one strided copy for K and one for V: the copies of
+    // small pageable head rows each cost the host about 10 us (16 of them for a 512-row board
+    // transaction: 206 us of its 671).  K's copy runs while V is staged.
+    const size_t head_bytes = (size_t)n * row_bytes, side = head_bytes * c->cfg.n_kv_heads;
+    if (2 * side <= kKvStageBytes) {
+        if (2 * side > c->kv_pinned_bytes) {
+            if (c->kv_pinned) (void)hipHostFree(c->kv_pinned);
+            c->kv_pinned = nullptr;
+            c->kv_pinned_bytes = 0;
+            if (hipHostMalloc((void**)&c->kv_pinned, 2 * side, 0) != hipSuccess) {
+                c->kv_pinned = nullptr;
+                return GQA_ERR_OOM;
+            }
+            c->kv_pinned_bytes = 2 * side;
+        }
+        HIP_TRY(hipEventRecord(c->ev_begin, c->stream));
+        const size_t dst = ((size_t)b * c->cfg.n_kv_heads * c->l_cap + start_pos) * D, pitch = c->l_cap * row_bytes;
+        const uint16_t* from[2] = {k, v};
+        uint16_t* to[2] = {c->k_cache + dst, c->v_cache + dst};
+        for (int i = 0; i < 2; ++i) {
+            uint8_t* stage = c->kv_pinned + i * side;
+            memcpy(stage, from[i], side);
+            if (head_bytes == pitch)
+                HIP_TRY(hipMemcpyAsync(to[i], stage, side, hipMemcpyHostToDevice, c->stream));
+            else
+                HIP_TRY(hipMemcpy2DAsync(to[i], pitch, stage, head_bytes, head_bytes, c->cfg.n_kv_heads,
+                                         hipMemcpyHostToDevice, c->stream));
+        }
+        return finish_sync(c);
+    }
     HIP_TRY(hipEventRecord(c->ev_begin, c->stream));
     for (int h = 0; h < c->cfg.n_kv_heads; ++h) {
         const size_t dst = (((size_t)b * c->cfg.n_kv_heads + h) * c->l_cap + start_pos) * D;
@@ -1657,8 +1725,18 @@ int gqa_submit(gqa_ctx* c, int32_t b, const uint16_t* q, int32_t q_len, int32_t 
     c->txn.causal = causal ? 1 : 0;
     const size_t qwords = (size_t)c->cfg.n_q_heads * q_len * c->cfg.head_dim;
     HIP_TRY(hipEventRecord(c->ev_t[0], c->stream));
-    HIP_TRY(hipMemcpyAsync(c->q_dev, q, qwords * 2, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    // Q goes through the output's pinned buffer, which holds nothing from here to the output's own copy (behind
+    // Q's on the stream): the runtime's staging of a pageable copy costs as much and, on a new stream, its
+    // allocation (0.7 ms).  Each part is on its way while the next is staged, and none is waited for.
+    if (c->q_in_flight) HIP_TRY(hipStreamSynchronize(c->stream));  // submitted again before it was started
+    c->q_in_flight = true;
+    const size_t bytes = qwords * 2;
+    const int parts = output_parts(bytes);
+    for (int i = 0; i < parts; ++i) {
+        const size_t at = output_part(bytes, parts, i), n = output_part(bytes, parts, i + 1) - at;
+        memcpy((uint8_t*)c->o_pinned + at, (const uint8_t*)q + at, n);
+        HIP_TRY(hipMemcpyAsync((uint8_t*)c->q_dev + at, (uint8_t*)c->o_pinned + at, n, hipMemcpyHostToDevice, c->stream));
+    }
     c->txn.valid = 1;
     return GQA_OK;
 }
@@ -1797,8 +1875,13 @@ int gqa_start(gqa_ctx* c) {
     c->v_cache = v_active;
     if (rc != GQA_OK) return rc;
     HIP_TRY(hipEventRecord(c->ev_t[2], c->stream));
-    const size_t owords = (size_t)c->cfg.n_q_heads * t.q_len * c->cfg.head_dim;
-    HIP_TRY(hipMemcpyAsync(c->o_pinned, c->o_dev, owords * 2, hipMemcpyDeviceToHost, c->stream));
+    const size_t bytes = (size_t)c->cfg.n_q_heads * t.q_len * c->cfg.head_dim * 2;
+    const int parts = output_parts(bytes);
+    for (int i = 0; i < parts; ++i) {
+        const size_t at = output_part(bytes, parts, i), n = output_part(bytes, parts, i + 1) - at;
+        HIP_TRY(hipMemcpyAsync((uint8_t*)c->o_pinned + at, (uint8_t*)c->o_dev + at, n, hipMemcpyDeviceToHost, c->stream));
+        if (i + 1 < parts) HIP_TRY(hipEventRecord(c->ev_part[i], c->stream));
+    }
     HIP_TRY(hipEventRecord(c->ev_t[3], c->stream));
     c->txn.running = 1;
     return GQA_OK;
@@ -1827,24 +1910,9 @@ int gqa_status(gqa_ctx* c, uint32_t* out_status) {
 int gqa_wait(gqa_ctx* c, int32_t timeout_ms) {
     if (!c) return GQA_ERR_NULL;
     if (!c->txn.running) return GQA_ERR_NO_TRANSACTION;  // nothing started (submitted or not)
-    struct timespec t0;
-    clock_gettime(CLOCK_MONOTONIC, &t0);
-    for (;;) {
-        hipError_t e = hipEventQuery(c->ev_t[3]);
-        if (e == hipSuccess) break;
-        if (e != hipErrorNotReady) {
-            last_hip_error(e, "hipEventQuery");
-            return GQA_ERR_HIP;
-        }
-        if (timeout_ms >= 0) {
-            struct timespec t1;
-            clock_gettime(CLOCK_MONOTONIC, &t1);
-            const double ms = (t1.tv_sec - t0.tv_sec) * 1e3 + (t1.tv_nsec - t0.tv_nsec) * 1e-6;
-            if (ms > timeout_ms) return GQA_ERR_TIMEOUT;
-        }
-        struct timespec nap = {0, 20000};
-        nanosleep(&nap, nullptr);
-    }
+    const int rc = wait_event(c->ev_t[3], timeout_ms);
+    if (rc != GQA_OK) return rc;
+    c->q_in_flight = false;
     float k_ms = 0.f, tot_ms = 0.f, copy_ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&k_ms, c->ev_t[1], c->ev_t[2]));
     HIP_TRY(hipEventElapsedTime(&tot_ms, c->ev_t[0], c->ev_t[3]));
@@ -1861,9 +1929,14 @@ int gqa_read_output(gqa_ctx* c, uint16_t* o, int64_t n_words) {
     if (!c->txn.running) return GQA_ERR_NO_TRANSACTION;
     const int64_t expect = (int64_t)c->cfg.n_q_heads * c->txn.q_len * c->cfg.head_dim;
     if (n_words != expect) return GQA_ERR_RESULT_LEN;
-    int rc = gqa_wait(c, -1);
-    if (rc != GQA_OK) return rc;
-    memcpy(o, c->o_pinned, (size_t)expect * 2);
+    const size_t bytes = (size_t)expect * 2;
+    const int parts = output_parts(bytes);
+    for (int i = 0; i < parts; ++i) {
+        const int rc = i + 1 < parts ? wait_event(c->ev_part[i], -1) : gqa_wait(c, -1);
+        if (rc != GQA_OK) return rc;
+        const size_t at = output_part(bytes, parts, i);
+        memcpy((uint8_t*)o + at, (uint8_t*)c->o_pinned + at, output_part(bytes, parts, i + 1) - at);
+    }
     return GQA_OK;
 }
 

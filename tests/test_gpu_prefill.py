@@ -537,3 +537,37 @@ def test_segment_workspace_stays_with_its_stream():
             for q, o in zip(qs, o_dev):
                 ref, _ = oracle_for(q, k, v, causal=True, q_pos_base=kv_len - q_len)
                 check_rows(o.cpu().numpy().view(np.uint16), None, ref, None)
+
+
+@pytest.mark.parametrize("L", [1, 63, 64, 301, 512])
+def test_transaction_staging(L):
+    """Q and the output share the context's pinned buffer, in up to four parts: a query submitted twice before the
+    start, an output read twice, a transaction started again, a K/V load between output and read-back (its own
+    staging), and with and without a timeout."""
+    rng = np.random.default_rng(5200 + L)
+    print(f"[staging] L={L}", flush=True)
+    q, q2 = bf16_normal(rng, (32, L, 128)), bf16_normal(rng, (32, L, 128))
+    k, v = bf16_normal(rng, (8, L, 128)), bf16_normal(rng, (8, L, 128))
+    with AttentionAccelerator() as acc:
+        acc.load_kv(k, v)
+        acc.submit_query(q2)
+        acc.submit_query(q)
+        acc.start()
+        acc.wait_done(q, k, v, L)
+        acc.load_kv(k, v)
+        first = acc.readback_o(L)
+        assert np.array_equal(acc.read_output(), first)
+        acc.start()
+        assert np.array_equal(acc.readback_o(L), first)
+        other = acc.run_attention(q2, k, v, timeout_ms=20000)
+        prof = acc.last_profile
+        assert prof.request_service_ms > 0 and prof.output_dma_transfer_ms > 0
+        again = acc.run_attention(q, k, v)
+        prof = acc.last_profile
+        assert prof.request_service_ms >= 0 and prof.output_dma_transfer_ms > 0
+        assert np.array_equal(again, first)
+        kr, vr = acc.read_kv(0, 0, L)
+    assert np.array_equal(kr, k) and np.array_equal(vr, v)
+    for out, qq in ((first, q), (other, q2)):
+        ref, _ = oracle_for(qq, k, v, causal=True)
+        check_rows(out, None, ref, None)
