@@ -67,7 +67,7 @@ extern "C" {
                                   the automatic plan's) splits; a last split of <= chunk/4 keys joins the one
                                   before it; 0 = auto: about 8 waves per CU, whole 16-key rounds per wave).
                                   The automatic plan does not split a (sequence, kv head) whose K/V take
-                                  at most 128 KiB.  Work-groups have 8 waves, or 4 when the 8-wave plan
+                                  at most 128 KiB (256 KiB from 32 of them on).  Work-groups have 8 waves, or 4 when the 8-wave plan
                                   has at most 8 work-groups (the automatic chunk is then planned for 4) */
 #define GQA_OPT_PROFILE      2 /* 1 = time every kernel launch with a HIP event pair bound to the launch
                                   (hipExtLaunchKernel; restarts the record).  Binding adds no GPU work
@@ -105,7 +105,7 @@ extern "C" {
  * finish merges the others' partials inside the decode launch (agent-scope atomics and a per-unit
  * arrival counter; one launch per step).  LAUNCH: a second, log-sum-exp merge launch.  AUTO (default):
  * FUSED while the split grid (sequences x kv heads x splits) is at most half the GPU's CU count and a
- * sequence has at most 16 splits -- every split ends with an L2 write-back of its XCD and an increment
+ * sequence has at most 32 splits -- every split ends with an L2 write-back of its XCD and an increment
  * of its sequence's counter, which saves the launch for short steps but slows the streaming of larger
  * grids more than a launch costs -- else LAUNCH.  An automatic plan of the shortest splits (one round
  * of every wave) that would need the merge launch takes splits twice as long where that lets AUTO fuse.

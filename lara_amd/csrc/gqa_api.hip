@@ -203,11 +203,17 @@ int plan_splits(int batch, int n_kv_heads, int n_cu, int waves) {
 // A (sequence, kv head) whose K/V take at most this many bytes is not split: one work-group streams
 // it in about a microsecond, less than merging splits costs (8 q / 2 kv heads, D 64, 256 keys = 64 KiB
 // per unit: 4.2 us of kernel in one split per unit against 4.8 us in four splits merged in-launch).
+// With kUnsplitUnits units and more the GPU has work enough without splits up to twice that (us a step over three
+// streams / on one, split against unsplit: 8 sequences of 300 keys, 32/8 heads of 128, 8.1 / 9.3 against 4.4 /
+// 6.0; 16 of 500 8.7 / 11.0 against 5.8 / 9.3; 40 of 600, 8/2 heads of 64, 8.1 / 9.1 against 4.4 / 6.4; but one of 500, 8
+// units, 4.3 / 7.0 against 4.4 / 9.1).
 constexpr int64_t kDecodeSplitMinBytes = 128 << 10;
+constexpr int kUnsplitUnits = 32;
 
 int plan_chunk(int batch, int n_kv_heads, int group, int n_cu, int max_len, int waves, int head_dim) {
     const int quantum = waves * decode_round_keys(group);
-    if ((int64_t)max_len * head_dim * 2 * 2 <= kDecodeSplitMinBytes)
+    const int64_t unit_bytes = (int64_t)max_len * head_dim * 2 * 2;
+    if (unit_bytes <= (batch * (int64_t)n_kv_heads >= kUnsplitUnits ? 2 : 1) * kDecodeSplitMinBytes)
         return std::max(quantum, (max_len + quantum - 1) / quantum * quantum);
     const int splits = plan_splits(batch, n_kv_heads, n_cu, waves);
     const int even = (max_len + splits - 1) / splits;
@@ -221,12 +227,12 @@ int plan_chunk(int batch, int n_kv_heads, int group, int n_cu, int max_len, int 
 // sequence's arrival counter, and the last one with an acquire (an L2 invalidate): that saves the
 // merge launch where the step is a short latency chain, but the L2 maintenance of many work-groups
 // slows the streaming of the others.  AUTO fuses up to kFusedMergeSplits splits per sequence while
-// the split grid fills at most half the CUs (measured, kernel time per step, fused vs launch: 4
+// the split grid fills at most half the CUs (16 of them until the plans below bounded the grid; measured, kernel time per step, fused vs launch: 4
 // work-groups (2 splits of 128 keys) 5.1 vs 8.1 us, 64 work-groups (8 splits of 512) 9.4 vs 11.7 us,
 // 32 q / 8 kv heads, one sequence of 2049 keys: 128 work-groups (16 splits of 128) 7.5 vs 8.6 us;
 // 256 work-groups: 8 splits of 16384 keys 314.1 vs 311.5 us, 4 of 8192 161 vs 160 us, 2 of 4096
 // 83-86 vs 81-82 us, 2 of 512 16.7 vs 16.1 us; 32 splits of 128 keys 9.4 vs 8.8 us).
-constexpr int kFusedMergeSplits = 16;
+constexpr int kFusedMergeSplits = 32;
 
 bool fuse_merge(int option, int units, int max_splits, int n_cu) {
     if (max_splits <= 1 || option == GQA_DECODE_MERGE_LAUNCH) return false;
@@ -247,6 +253,22 @@ bool fuse_merge(int option, int units, int max_splits, int n_cu) {
 // of 2049 keys, 8 fused splits of 256 8.50 against 16 of 128 and a launch 9.00).
 constexpr int64_t kSmallDecodeGrid = 8;
 
+// Two more ranges of the automatic plan, in splits of whole 64-key steps (us a step over three streams / on one,
+// before against after):
+//  - K/V of at most kFusedPlanBytes over at most kFusedPlanUnits units: about kFusedPlanGrid work-groups merged
+//    in-launch.  A grid that fills the CUs pays a merge launch, or an L2 write-back per work-group, for a
+//    stream of a few us: one sequence of 8000 keys, 8/2 heads of 64, 7.9 / 9.4 against 4.4 / 7.3 (62
+//    work-groups); 10 of 2000 8.1 / 9.1 against 5.2 / 8.0; 4 of 1000, 32/8 heads of 128, 7.1 / 9.1 against 6.0 / 9.0; 7
+//    of up to 3000, 32/2 heads of 64, 8.0 / 10.8 against 5.5 / 10.9.
+//  - up to kStreamPlanBytes over 8 units to kFusedPlanUnits, in splits of three rounds a wave and more:
+//    kStreamPlanGrid work-groups merged by a launch, which leaves room for the merge of the launch before: one of
+//    16000 keys, 32/8 heads of 128, 11.9 / 15.7 against 11.7 / 15.0; of 30000 20.0 / 23.7 against 18.9 / 23.1; of
+//    20000, 64/8 heads, 15.1 / 19.2 against 14.7 / 18.7; 4 of 4000 13.1 / 15.0 against 11.7 / 15.3.  (Shorter splits
+//    gained nothing; above, 530 MB: 79.2 / 85.4 on 256 work-groups, 75.9 / 97.6 on 128, every CU streams.)
+constexpr int64_t kFusedPlanBytes = 16 << 20, kStreamPlanBytes = 128 << 20;
+constexpr int kFusedPlanUnits = 32;
+constexpr double kFusedPlanGrid = 112.0 / 256, kStreamPlanGrid = 208.0 / 256;  // of the CUs
+
 struct DecodeShape {
     int chunk;
     int max_splits;
@@ -263,6 +285,18 @@ DecodeShape plan_decode_shape(int batch, int n_kv_heads, int group, int head_dim
     };
     const DecodeShape big = shape(kDecodeWaves);
     if (units * big.max_splits <= kSmallDecodeGrid) return shape(kDecodeWavesSmall);
+    const int64_t bytes = units * max_len * head_dim * 2 * 2;
+    if (chunk_opt <= 0 && merge_option == GQA_DECODE_MERGE_AUTO && big.max_splits > 1 && units <= kFusedPlanUnits &&
+        bytes <= kStreamPlanBytes) {
+        const bool fused = bytes <= kFusedPlanBytes;
+        const int grid = (int)((fused ? kFusedPlanGrid : kStreamPlanGrid) * n_cu);
+        const int splits = std::max(1, std::min(fused ? kFusedMergeSplits : INT_MAX, grid / (int)units));
+        const int shortest = kDecodeWaves * decode_round_keys(group);
+        const int even = ((max_len + splits - 1) / splits + kChunkOptionQuantum - 1) / kChunkOptionQuantum * kChunkOptionQuantum;
+        const DecodeShape s{std::max(shortest, even), decode_split_count(max_len, std::max(shortest, even)), kDecodeWaves};
+        if (fused ? s.max_splits > 1 && fuse_merge(merge_option, (int)units, s.max_splits, n_cu) : units >= 8 && s.chunk >= 3 * shortest)
+            return s;
+    }
     if (chunk_opt <= 0 && merge_option == GQA_DECODE_MERGE_AUTO && big.max_splits > 1 &&
         big.chunk == kDecodeWaves * decode_round_keys(group) &&
         !fuse_merge(merge_option, (int)units, big.max_splits, n_cu)) {

@@ -399,3 +399,28 @@ def test_decode_auto_plan_merges_small_grids_in_launch(B, hq, hkv, d, L, twice):
         assert decodes == 2
         if n_cu == 256:
             assert merges == 0, "the automatic plan took the merge launch"
+
+
+@pytest.mark.parametrize("B,hq,hkv,d,L,merges", [(1, 8, 2, 64, 8000, 0), (10, 8, 2, 64, 2000, 0), (4, 32, 8, 128, 1000, 0),
+                                                 (7, 32, 2, 64, 2999, 0), (8, 32, 8, 128, 300, 0), (16, 32, 8, 128, 500, 0),
+                                                 (1, 32, 8, 128, 16001, 2), (1, 64, 8, 128, 9973, 2), (3, 32, 8, 128, 5000, 2)])
+def test_decode_auto_plan_ranges(B, hq, hkv, d, L, merges):
+    """The automatic plan's ranges: small K/V in about 112 work-groups merged in-launch or, from 32 (sequence, kv
+    head) units on, unsplit; larger ones in about 208 merged by a launch; ragged lengths with splits in 64-key
+    steps, each step against the oracle, twice (the arrival counters reset)."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(900 + B * 10 + d + L)
+    lens = np.full(B, L, np.int32)
+    if B > 1:
+        lens[1:] = rng.integers(L // 2, L + 1, B - 1)
+        lens[-1] = 1
+    print(f"[plan] B={B} hq={hq} hkv={hkv} d={d} L={L}", flush=True)
+    with make_engine(B, hq, hkv, d, L) as eng:
+        kc, vc = fill_cache(eng, rng, B, hkv, d, lens, lcap=L)
+        _lib.check(eng._lib.gqa_set_option(eng._ctx, _lib.GQA_OPT_PROFILE, 1), "profile")
+        for _ in range(2):
+            q = bf16_normal(rng, (B, hq, d))
+            out, lse = eng.decode_step(q, lens, return_lse=True)
+            check_decode(out, lse, q, kc, vc, lens, None)
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            assert _merge_launches(eng) == (merges, 2)
