@@ -243,14 +243,23 @@ def test_layer_at_2048_tokens_sampled_rows():
         assert float(orc.row_ulp_error(out[:, r0:r0 + 64], chain).max()) <= 3.0, r0
 
 
+def assert_same_stage(a, b):
+    """Two stages whose products may be summed in different orders (the library's algorithm is each context's own
+    choice): a product near a rounding boundary goes one bf16 ulp either way, and RoPE carries both of a pair's
+    into each, rounding again."""
+    a, b = (orc.bf16_u16_to_fp32(t).astype(np.float64) for t in (a, b))
+    pair = np.maximum(np.hypot(b[..., 0::2], b[..., 1::2]), 2.0 ** -6).repeat(2, axis=-1).astype(np.float32)
+    assert np.all(np.abs(a - b) <= 3 * orc.bf16_ulp(pair))
+
+
 @pytest.mark.parametrize("hidden,L,hq,hkv,d", [(1024, 1, 8, 2, 128), (1024, 16, 8, 2, 64), (2048, 3, 16, 8, 128),
                                                (4096, 1, 32, 8, 128), (4096, 15, 32, 8, 128), (4096, 16, 32, 2, 64),
                                                (4096, 17, 32, 8, 128), (8192, 1, 64, 8, 128), (8192, 8, 64, 8, 128),
                                                (8192, 9, 8, 2, 128), (4096, 5, 1, 1, 64)])
 def test_few_tokens_stage(hidden, L, hq, hkv, d):
     """The one-launch stage (up to 16 tokens, 8 at hidden 8192; the others take the general one): the projection
-    within its fp32 bound, RMSNorm through it, RoPE word for word, and the same words from separate weights, on
-    a paged cache and where a misaligned x sends the call to the general path (its own bound)."""
+    within its fp32 bound, RMSNorm through it, RoPE word for word, and the same words from separate weights and on
+    a paged cache (the general stage: up to the order of its sums)."""
     print(f"[layer] few tokens hidden={hidden} L={L} hq={hq} hkv={hkv} d={d}", flush=True)
     rng = np.random.default_rng(hidden + L + d)
     x = bf16_normal(rng, (L, hidden), 3.0)
@@ -276,7 +285,11 @@ def test_few_tokens_stage(hidden, L, hq, hkv, d):
             err = np.abs(got - lo.project_exact(xin, w))
             assert np.all(err <= bound), float(np.max(err / bound))
     for a, b, c, e in zip(plain, fused, roped, paged):
-        assert np.array_equal(a, b) and np.array_equal(c, e)
+        if L <= (8 if hidden > 4096 else 16):
+            assert np.array_equal(a, b) and np.array_equal(c, e)
+        else:
+            assert_same_stage(a, b)
+            assert_same_stage(c, e)
     assert np.array_equal(roped[0], lo.apply_rope(normed[0], 70001))
     assert np.array_equal(roped[1], lo.apply_rope(normed[1], 60)) and np.array_equal(roped[2], normed[2])
 
@@ -301,6 +314,4 @@ def test_few_tokens_stage_keeps_the_general_calls():
             acc.layer_qkv_device(src.data_ptr(), L, hidden, *(t.data_ptr() for t in bufs), dst.data_ptr())
             torch.cuda.synchronize()
             got = host(dst).reshape(8, L, 128)
-            diff = np.abs(orc.bf16_u16_to_fp32(got).astype(np.float64) - orc.bf16_u16_to_fp32(want[0]))
-            # the two paths sum in different orders: one bf16 ulp, and one more through the rotation
-            assert np.all(diff <= 2 * orc.bf16_ulp(np.maximum(np.abs(orc.bf16_u16_to_fp32(want[0])), 2.0 ** -6)))
+            assert_same_stage(got, want[0])
