@@ -83,7 +83,8 @@ extern "C" {
 /* Prefill decomposition (GQA_OPT_PREFILL_KERNEL).  SHARED: a work-group per kv head and 8 tasks of 32
  * (query row, head) pairs shares each K/V tile over its GQA group; launches smaller than the GPU are
  * cut into KV segments merged by a second launch (GQA_OPT_PREFILL_WGS).  ROWS: a work-group per
- * (query head, 32-row block) whose waves split the keys and merge in LDS (one launch, no segments).
+ * (query head, or two of them where one each would take several rounds of the CUs; 32-row block) whose
+ * waves split the keys and merge in LDS (one launch, no segments).
  * PAIRED: SHARED whose work-groups each own a long and a short causal row block (last and first),
  * the short one's waves moving to the long one's keys once theirs end, so the work-groups of a causal
  * launch carry equal work (causal launches of group 4 with more than one row block, always planned in

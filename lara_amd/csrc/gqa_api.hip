@@ -413,31 +413,61 @@ int check_prefill_args(const gqa_ctx* c, int32_t b, int32_t q_len, int32_t q_pos
     return GQA_OK;
 }
 
+// The keys an average row of a launch sees.
+double prefill_avg_keys(int q_len, int kv_span, bool causal) {
+    return causal ? kv_span - 0.5 * std::min(q_len, kv_span) : kv_span;
+}
+
+// Whether the row-block kernel takes two query heads per work-group: a work-group of its own per head would need
+// more than one round of the CUs, and the rounds after the first are not made of the short first rows of a
+// causal block alone, which fill in behind the long ones (us on one stream, one head against two: 32/8 heads,
+// 257 rows 9.2 against 10.6, 320 9.3 against 9.6; 16/8, 640 10.5 against 11.4; but 257 after 500 15.9 against 14.3, 513 15.7
+// against 14.1).
+bool rows_two_heads(int q_len, int kv_span, bool causal, int group, int n_kv_heads, int head_dim, int n_cu) {
+    const double share = (double)((q_len + kPrefillRows - 1) / kPrefillRows) * group * n_kv_heads / n_cu;
+    return head_dim == 128 && group % 2 == 0 && share > 1.0 &&
+           share * prefill_avg_keys(q_len, kv_span, causal) >= 0.75 * kv_span;
+}
+
 // KV segments for a launch of the shared kernel whose grid without them (`base` work-groups) is smaller
 // than the GPU, or 0 where the row-block kernel is the faster one.  The estimates are us fitted to one
 // MI355X over 5 .. 1500 rows, 0 .. 20000 earlier keys, 8/8, 16/8, 32/8 and 64/8 heads of 128 and 32/8 and 8/2 of
 // 64, most within 15 % of what was measured.  A launch's own time (back to back on one stream):
 //   row blocks: 2 + 2.5 per dispatch round, and per 256 keys 1.13 (a CU's load path) or, where the
 //     work-groups fill the GPU, 1.4 per round (the L2s' rate);
+//   row blocks of two heads: 2 + 6 per dispatch round, and per 256 keys 1.67, or 1.85 where it takes several rounds
+//     (the longest rows' in the first, an average row's in later ones), or 2.1 per full round;
 //   shared: 4 + a 64-key block's 0.75 and 0.13 for each further task of the work-group; with segments 10 + 0.7
 //     per MB of fp32 partials (written and read) instead of 4.
 // And what it takes from launches on other streams: the larger of its time in 2.5 concurrent launches and
 // the CUs it holds (shared: the work-groups' share of the GPU times 4 + their blocks, + 0.3 per MB; with
 // segments 7.5 at least, the host's two launches).
+// (Row blocks of two heads: the share of a round they fill times 8 + 2.15 per 256 keys.)
 // Segments have to save 4 of the first (the second launch costs the host more than a stream shows) and
 // must not lose the second.  So rows stay for short histories (32/8 heads, 100 rows after 4000 keys: 25.1 us
 // against 26.5; 37 after 2000: 15.0 against 18.4) and segments win the long ones (8 after 4000: 22.3 -> 14.9;
 // 37 after 12000: 57.2 -> 28.1; 100 after 20000: 89.9 -> 49.8; 500 after 8000: 94.9 -> 74.3; 64/8, 100 after
-// 20000: 106.2 -> 77.9).
+// 20000: 106.2 -> 77.9).  Against row blocks of two heads, whose launches mostly take several rounds, several segments
+// have to be within 1.1 of the first, about what this estimate exceeds the measured by there, and save 5 % of the
+// second (513 rows after 6000: 64.0 / 101.4 -> 56.2 / 88.8 us; but 768 after 6000 89.0 / 106.0 in row blocks); one segment,
+// measured 4 above its estimate, within 1.2, and save 40 % (64/8, 500 rows: 16.8 / 18.4 -> 9.0 / 21.8; but 300
+// 10.1 / 14.3 against 6.7 / 16.1).
 int plan_shared_segments(int q_len, int kv_span, bool causal, int group, int n_kv_heads, int head_dim, int n_cu,
                          int max_segs) {
     const int base = prefill_shared_wgs(q_len, group, n_kv_heads);
     const int tasks = prefill_tasks_per_wg(q_len, group);
     const double per_key = head_dim > 64 ? 1.0 : 0.65;  // of the work that grows with the keys
-    const double avg_keys = causal ? kv_span - 0.5 * std::min(q_len, kv_span) : kv_span;
+    const double avg_keys = prefill_avg_keys(q_len, kv_span, causal);
     const double share = (double)((q_len + kPrefillRows - 1) / kPrefillRows) * group * n_kv_heads / n_cu;
-    const double rows_us = 2.0 + 2.5 * std::max(1.0, share) + per_key * std::max(1.13 * kv_span, 1.4 * share * avg_keys) / 256;
-    const double rows_gpu_us = std::max(0.4, 1.05 * std::min(1.0, share)) * rows_us;
+    double rows_us = 2.0 + 2.5 * std::max(1.0, share) + per_key * std::max(1.13 * kv_span, 1.4 * share * avg_keys) / 256;
+    double rows_gpu_us = std::max(0.4, 1.05 * std::min(1.0, share)) * rows_us;
+    const bool two_heads = rows_two_heads(q_len, kv_span, causal, group, n_kv_heads, head_dim, n_cu);
+    if (two_heads) {
+        const double rounds = std::ceil(share / 2);
+        rows_us = 2.0 + 6.0 * std::max(1.0, share / 2) +
+                  std::max((rounds > 1 ? 1.85 : 1.67) * (kv_span + (rounds - 1) * avg_keys), 2.1 * share / 2 * avg_keys) / 256;
+        rows_gpu_us = std::max(0.4 * rows_us, share / 2 * (8.0 + 2.15 * avg_keys / 256));
+    }
     const double block_us = per_key * (0.75 + 0.13 * (tasks - 1));
     const int blocks = (kv_span + 63) / 64;
     const double partial_mb = 1e-6 * q_len * group * n_kv_heads * (head_dim + 2) * 4;
@@ -448,8 +478,9 @@ int plan_shared_segments(int q_len, int kv_span, bool causal, int group, int n_k
         const double us = (segs > 1 ? 10.0 : 4.0) + 0.7 * mb + loop_us;
         if (segs > 1 && rows_gpu_us < 7.5) break;  // the host's time for two launches
         const double gpu_us = std::max(0.4 * us, 1.05 * ((double)(base * segs) / n_cu * (4.0 + loop_us) + 0.3 * mb));
-        if (us + (segs > 1 ? 4.0 : 0.0) < best_us && gpu_us <= rows_gpu_us) {
-            best_us = us + (segs > 1 ? 4.0 : 0.0);
+        const double cost = two_heads ? (segs > 1 ? us / 1.1 : (us + 4.0) / 1.2) : segs > 1 ? us + 4.0 : us;
+        if (cost < best_us && gpu_us <= (two_heads ? (segs > 1 ? 0.95 : 0.6) : 1.0) * rows_gpu_us) {
+            best_us = cost;
             best = segs;
         }
     }
@@ -565,6 +596,7 @@ int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_p
     a.part_o = c->pre_ws;
     a.part_ml = c->pre_ws + (size_t)plan.n_segs * c->cfg.n_q_heads * q_len * c->cfg.head_dim;
     if (rows) {
+        a.rows_heads = rows_two_heads(q_len, kv_span, causal != 0, c->group, c->cfg.n_kv_heads, c->cfg.head_dim, c->n_cu) ? 2 : 1;
         HIP_TRY(launch_prefill_rows(c->cfg.head_dim, a, timed(c, GQA_TIMER_PREFILL, s)));
         c->last_prefill_kernel = GQA_PREFILL_KERNEL_ROWS;
         c->last_prefill_segs = 1;

@@ -131,6 +131,7 @@ struct PrefillArgs {
     int32_t n_segs;         // KV segments (grid z); 1 = write the output directly
     float* part_o;          // [n_segs][H_q][q_len][D] fp32: the segment's un-normalised O
     float* part_ml;         // [n_segs][H_q][q_len][2] (running max in log2 units, sum l)
+    int32_t rows_heads;     // row-block kernel: query heads per work-group (1, or 2 at D = 128 and an even group)
     const uint16_t* zero_row;  // >= D zero words: the source of K/V rows past kv_len
     // Paged cache: block_table is sequence b's row of page indices (-1 = unmapped, read as
     // zero_row, never written), kc/vc the pools [n_pages][H_kv][2^page_shift][D]; nullptr =

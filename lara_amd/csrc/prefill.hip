@@ -830,7 +830,7 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_kernel(PrefillArgs a) {
 
 // ---- Row-block prefill for launches too small to fill the GPU ------------------------------
 //
-// One work-group per (query head, 32-row block): a 256-row chunk over 32 query heads is 256
+// One work-group per (query head or pair of heads, 32-row block): a 256-row chunk over 32 query heads is 256
 // work-groups, one per CU, with no KV segments across work-groups and so no partials and no merge
 // launch.  The NW = 8 waves (two per SIMD) take the row block's 32-key blocks in turn (wave w:
 // blocks w, w+8, ...), each streaming its own K and V tile (one of each, refilled as soon as it has
@@ -842,25 +842,34 @@ __global__ __launch_bounds__(kWaves * 64) void prefill_kernel(PrefillArgs a) {
 // 16-key k-steps per 32-dim tile).
 constexpr int kRowBN = 32;  // keys per block
 
-// NW waves per work-group take the row block's key blocks in turn.
-template <int D, bool PAGED, int NW>
+// NW waves per work-group take the row block's key blocks in turn, for HT query heads of the kv head at once.
+// With one head a work-group is bound by its CU's load path (128 KiB per 256 keys at D = 128: 1.3 us), so a
+// launch of more work-groups than CUs reads the same K/V over that path once more per round.  With two heads each
+// tile read serves both (1.7 us per 256 keys for both, the CU's LDS: 48 KiB moved per 32 keys): their 128 O
+// registers leave no room for Q^T, which is read from LDS beside K, and a head's arithmetic and its order are
+// the same, word for word.  us a launch over three streams / on one, 32/8 heads of 128, one head -> two: 512 rows
+// 11.6 / 12.6 -> 9.2 / 11.7; 512 after 1536 26.3 / 28.0 -> 20.6 / 23.7; 288 after 2000 18.9 / 29.8 -> 14.2 / 23.8; 900 after 2000
+// 60.0 / 66.6 -> 47.1 / 52.5.  (Within one round they only give CUs to other streams: 256 rows after 1792 15.4 / 17.0
+// -> 11.6 / 22.2.  At D = 64 the load path is no bound: 700 rows 7.7 / 10.7 -> 9.3 / 12.0.)
+template <int D, bool PAGED, int NW, int HT>
 __global__ __launch_bounds__(NW * 64) void prefill_rows_kernel(PrefillArgs a) {
     constexpr int kRowWaves = NW;
     constexpr int NCH = D / 8;         // 16-byte chunks per K/V row
     constexpr int KSTEPS = D / 16;     // QK k-steps
     constexpr int MT = D / 32;         // PV result tiles (32 dims each)
     constexpr int TILE = kRowBN * NCH; // 16-byte chunks per K (or V) tile
-    constexpr int KA = KSTEPS > 3 ? 3 : KSTEPS - 1;  // K fragment reads in flight ahead of their MFMA
+    constexpr int KA = HT > 1 ? 2 : KSTEPS > 3 ? 3 : KSTEPS - 1;  // K fragment reads in flight ahead of their MFMA
     constexpr int VA = 2;                            // V^T steps read ahead of their MFMA
     constexpr int DMA = TILE / 64;     // direct-to-LDS loads per lane per tile
     static_assert(DMA >= 1 && DMA * 64 == TILE, "tile shape");
-    static_assert(D * kRows * 4 <= 2 * TILE * 16, "a wave's O^T fits its tiles");
+    constexpr bool Q_LDS = HT > 1;     // Q^T is read from LDS per block (of one head: kept in VGPRs)
+    static_assert(D * kRows * 4 <= 2 * TILE * 16, "a head's O^T fits the wave's tiles");
 
     // Per wave: one K and one V tile, reused for the wave's O^T after the loop, and its rows' (m, l);
     // the row block's Q, loaded once for all waves.
     __shared__ __attribute__((aligned(16))) u32x4 lds[kRowWaves][2][TILE];
-    __shared__ float lds_ml[kRowWaves][2][kRows];
-    __shared__ __attribute__((aligned(16))) u32x4 lds_q[TILE];
+    __shared__ float lds_ml[HT][kRowWaves][2][kRows];
+    __shared__ __attribute__((aligned(16))) u32x4 lds_q[HT][TILE];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -868,10 +877,10 @@ __global__ __launch_bounds__(NW * 64) void prefill_rows_kernel(PrefillArgs a) {
     const int h = blockIdx.x;  // kv head
     const int G = a.n_q_heads / a.n_kv_heads;
     const int n_rb = (a.q_len + kRows - 1) / kRows;
-    const int g = blockIdx.y % G;
+    const int sets = G / HT;  // of HT heads
     // Causal row blocks grow in work with their index: the largest are dispatched first.
-    const int rb = a.causal ? n_rb - 1 - (int)(blockIdx.y / G) : (int)(blockIdx.y / G);
-    const int hq = h * G + g;
+    const int rb = a.causal ? n_rb - 1 - (int)(blockIdx.y / sets) : (int)(blockIdx.y / sets);
+    const int hq = h * G + (int)(blockIdx.y % sets) * HT;  // the first head
 
     int kv_hi = a.kv_len;  // keys the row block needs: [0, kv_hi)
     if (a.causal) kv_hi = min(kv_hi, a.q_pos_base + min(a.q_len, (rb + 1) * kRows) - 1 - a.kv_pos_base + 1);
@@ -903,13 +912,17 @@ __global__ __launch_bounds__(NW * 64) void prefill_rows_kernel(PrefillArgs a) {
     // come from one contiguous run -- the cache, or the rows this launch appends -- takes a
     // wave-uniform base and these fixed offsets; a block that straddles the appended rows or ends
     // past kv_len (zero row there: stale words may be NaN) picks each lane's source.
-    uint32_t koff[DMA], voff[DMA];
+    // (Load i covers keys i*KPL .. +KPL-1.  With two heads, short of registers, the offsets that repeat are kept
+    // once: K's swizzle repeats every 16 keys, V's with every load.)
+    constexpr int KPL = 64 / NCH;
+    constexpr int KP = Q_LDS && 16 / KPL < DMA ? 16 / KPL : DMA, VP = Q_LDS ? 1 : DMA;
+    static_assert(!Q_LDS || KPL % 4 == 0, "whole periods of V's swizzle per load");
+    uint32_t koff[KP], voff[VP];
 #pragma unroll
     for (int i = 0; i < DMA; ++i) {
-        const int slot = i * 64 + lane;
-        const int key = slot / NCH;
-        koff[i] = 16u * (uint32_t)(key * NCH + ((slot % NCH) ^ k_swz<NCH>(key)));
-        voff[i] = 16u * (uint32_t)(key * NCH + ((slot % NCH) ^ v_swz<D>(key)));
+        const int key = i * KPL + lane / NCH;
+        if (i < KP) koff[i] = 16u * (uint32_t)(key * NCH + ((lane % NCH) ^ k_swz<NCH>(key)));
+        if (i < VP) voff[i] = 16u * (uint32_t)(key * NCH + ((lane % NCH) ^ v_swz<D>(key)));
     }
     const int new_end = has_new ? a.new_begin + a.n_new : 0;
     // pr: paged, the block's page row (paged_row_uniform of j0, looked up by the caller ahead of
@@ -935,55 +948,72 @@ __global__ __launch_bounds__(NW * 64) void prefill_rows_kernel(PrefillArgs a) {
         if (krow != nullptr) {
             const uint64_t base = uniform_address(kv ? vrow : krow);
 #pragma unroll
-            for (int i = 0; i < DMA; ++i) dma16_sbase(base, kv ? voff[i] : koff[i], lds_addr(&lds[wave][kv][i * 64]));
+            for (int i = 0; i < DMA; ++i)
+                dma16_sbase(base + (kv ? i / VP * VP : i / KP * KP) * 1024, kv ? voff[i % VP] : koff[i % KP],
+                            lds_addr(&lds[wave][kv][i * 64]));
             return;
         }
-        const int64_t pr0 = pr;
-#pragma unroll
+        // (With two heads: rolled up, and from a lane number of its own, so that nothing of it is kept in registers.
+        // With one head unrolled: around an inner loop the compiler does not peel the key loop's first block.)
+        int own_lane = lane;
+        if constexpr (Q_LDS) asm volatile("" : "+v"(own_lane));
+        constexpr int kUnroll = Q_LDS ? 1 : DMA;
+#pragma unroll kUnroll
         for (int i = 0; i < DMA; ++i) {
-            const int rel = (int)(koff[i] >> 4) / NCH;  // key of this lane's slot within the block
+            const int rel = i * KPL + own_lane / NCH;  // key of this lane's slot within the block
             const int row_idx = j0 + rel;
-            const uint32_t kc_off = koff[i] - 16u * (uint32_t)(rel * NCH);  // chunk offset within the row
-            const uint32_t vc_off = voff[i] - 16u * (uint32_t)(rel * NCH);
+            const int chunk = (own_lane % NCH) ^ (kv ? v_swz<D>(rel) : k_swz<NCH>(rel));
             const u32x4* src;
             const unsigned r_new = (unsigned)(row_idx - a.new_begin);
-            if (row_idx >= a.kv_len || (PAGED && pr0 < 0)) {
+            if (row_idx >= a.kv_len || (PAGED && pr < 0)) {
                 src = zero;
             } else if (has_new && r_new < (unsigned)a.n_new) {
                 src = (kv ? vn : kn) + (size_t)r_new * NCH;
             } else if constexpr (PAGED) {
-                src = (kv ? vg : kg) + (size_t)(pr0 + rel) * NCH;
+                src = (kv ? vg : kg) + (size_t)(pr + rel) * NCH;
             } else {
                 src = (kv ? vg : kg) + (size_t)row_idx * NCH;
             }
-            dma16(reinterpret_cast<const uint8_t*>(src) + (kv ? vc_off : kc_off), lds_addr(&lds[wave][kv][i * 64]));
+            dma16(src + chunk, lds_addr(&lds[wave][kv][i * 64]));
         }
     };
 
     // Operand addresses in this wave's tiles.
-    uint32_t kaddr[KSTEPS];
+    // K: row `col`, chunk 2 ks + half, XOR-swizzled (step ks: bits of the chunk apart from half's); V^T: the tile's
+    // dims likewise.  With one head every address is kept, with two the bases.
+    const uint32_t kcol = 16u * (uint32_t)(col * NCH + (half ^ k_swz<NCH>(col)));
+    const uint32_t ktile = lds_addr(&lds[wave][0][0]);
+    const int key_off = (lane & 15) >> 2, dim0 = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    const uint32_t vcol = (uint32_t)((key_off + 4 * half) * (D * 2) + (((dim0 >> 3) ^ v_swz<D>(key_off)) << 4) + (((dim0 >> 2) & 1) << 3));
+    const uint32_t vtile = lds_addr(&lds[wave][1][0]);
+    uint32_t kkept[Q_LDS ? 1 : KSTEPS], vkept[Q_LDS ? 1 : MT];
+    if constexpr (!Q_LDS) {
 #pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks)
-        kaddr[ks] = lds_addr(&lds[wave][0][0]) + 16u * (uint32_t)(col * NCH + ((2 * ks + half) ^ k_swz<NCH>(col)));
-    uint32_t vaddr[MT];
-    {
-        const int key_off = (lane & 15) >> 2;
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+            kkept[ks] = ktile + (kcol ^ (uint32_t)(32 * ks));
+            asm volatile("" : "+v"(kkept[ks]));  // (not computed again at each use)
+        }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            const int dim = mt * 32 + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-            vaddr[mt] = lds_addr(&lds[wave][1][0]) + (uint32_t)((key_off + 4 * half) * (D * 2) +
-                                                                   (((dim >> 3) ^ v_swz<D>(key_off)) << 4) +
-                                                                   (((dim >> 2) & 1) << 3));
+            vkept[mt] = vtile + (vcol ^ (uint32_t)(64 * mt));
+            asm volatile("" : "+v"(vkept[mt]));
         }
     }
+    auto kaddr = [&](auto ks) { return Q_LDS ? ktile + (kcol ^ (uint32_t)(32 * ks.value)) : kkept[Q_LDS ? 0 : ks.value]; };
+    auto vaddr = [&](auto mt) { return Q_LDS ? vtile + (vcol ^ (uint32_t)(64 * mt.value)) : vkept[Q_LDS ? 0 : mt.value]; };
 
-    f32x16 o[MT];
+    f32x16 o[HT][MT];
+    float m_run[HT];   // running max (log2 units) of this lane's row
+    float l_lane[HT];  // this lane's half of the running sum
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int n = 0; n < HT; ++n) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) o[mt][i] = 0.f;
-    float m_run = -INFINITY;  // running max (log2 units) of this lane's row
-    float l_lane = 0.f;       // this lane's half of the running sum
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[n][mt][i] = 0.f;
+        m_run[n] = -INFINITY;
+        l_lane[n] = 0.f;
+    }
     constexpr float kLazyLog2 = 8.0f;  // the reference max moves only when passed by more than this
     constexpr float kFreeSum = 65536.0f;  // 2^16, as in prefill_kernel
     const float c = a.scale_log2;
@@ -1010,14 +1040,14 @@ __global__ __launch_bounds__(NW * 64) void prefill_rows_kernel(PrefillArgs a) {
     // Then Q^T's rows (row `row`, dims 16*ks + 8*half .. +7) and the wave's first K and V tiles.
     // Q of the row block goes to LDS once (the K tile's swizzled layout, rows past q_len from the zero
     // row), each lane one 16-byte chunk, instead of every wave loading all 32 rows.
-    for (int base = wave * 64; base < TILE; base += kRowWaves * 64) {  // base is wave-uniform
-        const int slot = base + lane;
+    for (int base = wave * 64; base < HT * TILE; base += kRowWaves * 64) {  // base is wave-uniform
+        const int slot = (base + lane) % TILE, head = hq + base / TILE;
         const int qrow = slot / NCH;
         const int chunk = (slot % NCH) ^ k_swz<NCH>(qrow);
         const u32x4* src = rb * kRows + qrow < a.q_len
-                               ? reinterpret_cast<const u32x4*>(a.q + ((size_t)hq * a.q_len + rb * kRows + qrow) * D) + chunk
+                               ? reinterpret_cast<const u32x4*>(a.q + ((size_t)head * a.q_len + rb * kRows + qrow) * D) + chunk
                                : zero + chunk;
-        dma16(src, lds_addr(&lds_q[base]));
+        dma16(src, lds_addr(&lds_q[0][0] + base));
     }
     // Loads complete in issue order, so at most V(0)'s DMA loads in flight means the appended word,
     // Q and K(0) have landed: V(0) lands behind the first S^T (the loop waits for it before PV).
@@ -1031,11 +1061,10 @@ __global__ __launch_bounds__(NW * 64) void prefill_rows_kernel(PrefillArgs a) {
     vm_wait<DMA>(app_k, app_v);
     __syncthreads();  // every wave's share of Q is in LDS
     u32x4 qb[KSTEPS];  // Q^T operand: row `row`, dims 16*ks + 8*half .. +7
-    {
-        const uint32_t qbase = lds_addr(&lds_q[0]);
+    const uint32_t qtile = lds_addr(&lds_q[0][0]);  // (the K tile's layout)
+    if constexpr (!Q_LDS) {
 #pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks)
-            qb[ks] = lds_read128(qbase + 16u * (uint32_t)(col * NCH + ((2 * ks + half) ^ k_swz<NCH>(col))));
+        for (int ks = 0; ks < KSTEPS; ++ks) qb[ks] = lds_read128(qtile + (kcol ^ (uint32_t)(32 * ks)));
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     if (app_first < app_words) {
@@ -1068,20 +1097,38 @@ __global__ __launch_bounds__(NW * 64) void prefill_rows_kernel(PrefillArgs a) {
 
         // ---- S^T = K . Q^T (raw scores): one 32x32 tile, K fragments read KA steps ahead ----
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        f32x16 sacc;
+        f32x16 sacc[HT];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sacc[i] = 0.f;
-        u32x4 kf[KSTEPS];
-        static_for<KA>([&](auto c) { kf[decltype(c)::value] = lds_read128(kaddr[decltype(c)::value]); });
+        for (int n = 0; n < HT; ++n)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sacc[n][i] = 0.f;
+        u32x4 kf[KSTEPS], qf[HT][KSTEPS];
+        auto read_k = [&](auto step_c) {
+            constexpr int ks = decltype(step_c)::value;
+            kf[ks] = lds_read128(kaddr(step_c));
+            if constexpr (Q_LDS) {
+                const uint32_t qa = qtile + (kcol ^ (uint32_t)(32 * ks));
+                static_for<HT>([&](auto n) { qf[decltype(n)::value][ks] = lds_read128<decltype(n)::value * TILE * 16>(qa); });
+            }
+        };
+        static_for<KA>([&](auto c) { read_k(c); });
         static_for<KSTEPS>([&](auto c) {
             constexpr int ks = decltype(c)::value;
-            if constexpr (ks + KA < KSTEPS) {
-                kf[ks + KA] = lds_read128(kaddr[ks + KA]);
-                lgkm_wait1<KA>(kf[ks]);  // reads complete in order: at most the KA later ones remain
+            if constexpr (ks + KA < KSTEPS) read_k(std::integral_constant<int, ks + KA>{});
+            // reads complete in order: at most those of the later steps remain
+            constexpr int later = ks + KA < KSTEPS ? KA : KSTEPS - 1 - ks;
+            if constexpr (Q_LDS) {
+                lgkm_wait<(HT + 1) * later + HT - 1>(kf[ks], qf[0][ks]);
+                sacc[0] = mfma32(kf[ks], qf[0][ks], sacc[0]);
+                static_for<HT - 1>([&](auto n_c) {
+                    constexpr int n = decltype(n_c)::value + 1;
+                    lgkm_wait1<(HT + 1) * later + HT - 1 - n>(qf[n][ks]);
+                    sacc[n] = mfma32(kf[ks], qf[n][ks], sacc[n]);
+                });
             } else {
-                lgkm_wait1<KSTEPS - 1 - ks>(kf[ks]);
+                lgkm_wait1<later>(kf[ks]);
+                sacc[0] = mfma32(kf[ks], qb[ks], sacc[0]);
             }
-            sacc = mfma32(kf[ks], qb[ks], sacc);
         });
         // Every read of the K tile is complete (lgkmcnt(0) above): it takes the next block's K.
         if (more) issue(j0 + kRowWaves * kRowBN, 0, pr_next);
@@ -1089,55 +1136,58 @@ __global__ __launch_bounds__(NW * 64) void prefill_rows_kernel(PrefillArgs a) {
         // ---- online softmax (log2 domain, scale folded into the exponent) ----
         const bool need_mask =
             (j0 + kRowBN > a.kv_len) || (a.causal && a.kv_pos_base + j0 + kRowBN - 1 > a.q_pos_base + rb * kRows);
-        if (need_mask) {
-            const int d = key_lim - (j0 + 4 * half);  // key j0 + 4*half + c is valid iff c < d
+        u32x4 pb[HT][2];  // P^T operand of the two PV k-steps (keys 0-15, 16-31 of the block)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) sacc[i] = 8 * (i >> 2) + (i & 3) < d ? sacc[i] : -INFINITY;
-        }
-        float psum = 0.f;
-        u32x4 pb[2];  // P^T operand of the two PV k-steps (keys 0-15, 16-31 of the block)
-        auto weights = [&]() __attribute__((always_inline)) {
-            const float nm = (m_run == -INFINITY) ? 0.f : -m_run;
-            psum = 0.f;
+        for (int n = 0; n < HT; ++n) {
+            if (need_mask) {
+                const int d = key_lim - (j0 + 4 * half);  // key j0 + 4*half + c is valid iff c < d
 #pragma unroll
-            for (int a2 = 0; a2 < 2; ++a2) {
-                float p[8];
+                for (int i = 0; i < 16; ++i) sacc[n][i] = 8 * (i >> 2) + (i & 3) < d ? sacc[n][i] : -INFINITY;
+            }
+            float psum = 0.f;
+            auto weights = [&]() __attribute__((always_inline)) {
+                const float nm = (m_run[n] == -INFINITY) ? 0.f : -m_run[n];
+                psum = 0.f;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    p[j] = __builtin_amdgcn_exp2f(fmaf(sacc[8 * a2 + j], c, nm));
-                    psum += p[j];
+                for (int a2 = 0; a2 < 2; ++a2) {
+                    float p[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        p[j] = __builtin_amdgcn_exp2f(fmaf(sacc[n][8 * a2 + j], c, nm));
+                        psum += p[j];
+                    }
+                    pb[n][a2] = u32x4{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
+                                      pack_bf16x2(p[6], p[7])};
                 }
-                pb[a2] = u32x4{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
-                               pack_bf16x2(p[6], p[7])};
+            };
+            // As in prefill_kernel: against the reference max directly once every row has one; the
+            // block's own max only where a lane's weights sum past kFreeSum or overflow.
+            bool need_max = __ballot(m_run[n] == -INFINITY) != 0;
+            if (!need_max) {
+                weights();
+                need_max = __ballot(!(psum <= kFreeSum)) != 0;  // also true for inf and NaN
             }
-        };
-        // As in prefill_kernel: against the reference max directly once every row has one; the
-        // block's own max only where a lane's weights sum past kFreeSum or overflow.
-        bool need_max = __ballot(m_run == -INFINITY) != 0;
-        if (!need_max) {
-            weights();
-            need_max = __ballot(!(psum <= kFreeSum)) != 0;  // also true for inf and NaN
-        }
-        if (need_max) {
-            float mx = -INFINITY;
+            if (need_max) {
+                float mx = -INFINITY;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[i]);
-            mx = pair_max32(mx);
-            const float bm = mx * c;
-            const bool grow = bm > m_run + kLazyLog2;
-            if (__ballot(grow) != 0) {
-                const float m_new = grow ? bm : m_run;
-                const float corr = (m_run == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
-                m_run = m_new;
-                l_lane *= corr;
+                for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[n][i]);
+                mx = pair_max32(mx);
+                const float bm = mx * c;
+                const bool grow = bm > m_run[n] + kLazyLog2;
+                if (__ballot(grow) != 0) {
+                    const float m_new = grow ? bm : m_run[n];
+                    const float corr = (m_run[n] == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_run[n] - m_new);
+                    m_run[n] = m_new;
+                    l_lane[n] *= corr;
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
+                    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) o[mt][i] *= corr;
+                        for (int i = 0; i < 16; ++i) o[n][mt][i] *= corr;
+                }
+                weights();
             }
-            weights();
+            l_lane[n] += psum;
         }
-        l_lane += psum;
 
         // ---- O^T += V^T . P^T, transposing V reads one step ahead ----
         if (more) wait_vmcnt<DMA>(); else wait_vmcnt<0>();  // V(t) landed; K(t+1) may still be in flight
@@ -1146,7 +1196,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_rows_kernel(PrefillArgs a) {
         auto read_v = [&](auto step_c) {
             constexpr int i = decltype(step_c)::value;
             constexpr int kb = 16 * (i & 1);  // step's key base within the block (half adds 4)
-            const uint32_t va = vaddr[i >> 1];
+            const uint32_t va = vaddr(std::integral_constant<int, (i >> 1)>{});
             vf[i][0] = lds_read_tr64<kb * (D * 2)>(va);
             vf[i][1] = lds_read_tr64<(kb + 8) * (D * 2)>(va);
         };
@@ -1160,93 +1210,97 @@ __global__ __launch_bounds__(NW * 64) void prefill_rows_kernel(PrefillArgs a) {
                 lgkm_wait<2 * (PV - 1 - i)>(vf[i][0], vf[i][1]);
             }
             const u32x4 vw = {vf[i][0].x, vf[i][0].y, vf[i][1].x, vf[i][1].y};
-            o[i >> 1] = mfma32(vw, pb[i & 1], o[i >> 1]);
+#pragma unroll
+            for (int n = 0; n < HT; ++n) o[n][i >> 1] = mfma32(vw, pb[n][i & 1], o[n][i >> 1]);
         });
         // Every read of the V tile is complete (lgkmcnt(0) above): it takes the next block's V.
         if (more) issue(j0 + kRowWaves * kRowBN, 1, pr_next);
     }
 
-    // ---- merge the waves: each writes (O^T [D][32 rows], m, l) to its own ring (no DMA pending) ----
+    // ---- merge the waves, head after head: each writes (O^T [D][32 rows], m, l) to its own tiles (no DMA
+    // pending) ----
     // O^T goes to LDS row-major, [32 rows][D] fp32, as 16-byte granules (four dims) XOR-swizzled by
     // the row so that neither the writes here nor the reads below conflict on banks.
-    const float l_row = l_lane + half_swap(l_lane, half);
     constexpr int GR = D / 4;  // granules per row
-    float4* mo = reinterpret_cast<float4*>(&lds[wave][0][0]);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-            const int gran = 8 * mt + 2 * i4 + half;  // dims 4*gran .. +3 = mt*32 + 8*i4 + 4*half + 0..3
-            mo[col * GR + (gran ^ (col % GR))] =
-                make_float4(o[mt][4 * i4], o[mt][4 * i4 + 1], o[mt][4 * i4 + 2], o[mt][4 * i4 + 3]);
-        }
-    if (half == 0) {
-        lds_ml[wave][0][col] = m_run;
-        lds_ml[wave][1][col] = l_row;
-    }
-    __syncthreads();
     // The work-group's threads over 32 rows: each takes DPT dims (at least 8, one 16-byte store).
     constexpr int NDG = kRowWaves * 64 / kRows;
     constexpr int DPT = D / NDG >= 8 ? D / NDG : 8;
     const int r = tid & 31;
     const int dg = tid >> 5;
     const int out_row = rb * kRows + r;
-    if (out_row >= a.q_len || dg * DPT >= D) return;
-    float wt[kRowWaves];
-    float M = -INFINITY, L = 0.f;
 #pragma unroll
-    for (int w = 0; w < kRowWaves; ++w) M = fmaxf(M, lds_ml[w][0][r]);
+    for (int n = 0; n < HT; ++n) {
+        if (n > 0) __syncthreads();  // the head before has been read
+        float4* mo = reinterpret_cast<float4*>(&lds[wave][0][0]);
 #pragma unroll
-    for (int w = 0; w < kRowWaves; ++w) {
-        const float mw = lds_ml[w][0][r];
-        wt[w] = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);
-        L = fmaf(wt[w], lds_ml[w][1][r], L);
-    }
-    const float inv = L > 0.f ? 1.f / L : 0.f;
-    uint16_t* orow = a.out + ((size_t)hq * a.q_len + out_row) * D + dg * DPT;
+        for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int d8 = 0; d8 < DPT; d8 += 8) {
-        float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        const int g0 = (dg * DPT + d8) / 4;  // first of the two granules of these eight dims
+            for (int i4 = 0; i4 < 4; ++i4) {
+                const int gran = 8 * mt + 2 * i4 + half;  // dims 4*gran .. +3 = mt*32 + 8*i4 + 4*half + 0..3
+                mo[col * GR + (gran ^ (col % GR))] =
+                    make_float4(o[n][mt][4 * i4], o[n][mt][4 * i4 + 1], o[n][mt][4 * i4 + 2], o[n][mt][4 * i4 + 3]);
+            }
+        const float l_row = l_lane[n] + half_swap(l_lane[n], half);
+        if (half == 0) {
+            lds_ml[n][wave][0][col] = m_run[n];
+            lds_ml[n][wave][1][col] = l_row;
+        }
+        __syncthreads();
+        if (out_row >= a.q_len || dg * DPT >= D) continue;
+        float wt[kRowWaves];
+        float M = -INFINITY, L = 0.f;
+#pragma unroll
+        for (int w = 0; w < kRowWaves; ++w) M = fmaxf(M, lds_ml[n][w][0][r]);
 #pragma unroll
         for (int w = 0; w < kRowWaves; ++w) {
-            const float4* wo = reinterpret_cast<const float4*>(&lds[w][0][0]) + r * GR;
-            const float4 x0 = wo[g0 ^ (r % GR)];
-            const float4 x1 = wo[(g0 + 1) ^ (r % GR)];
-            v[0] = fmaf(wt[w], x0.x, v[0]);
-            v[1] = fmaf(wt[w], x0.y, v[1]);
-            v[2] = fmaf(wt[w], x0.z, v[2]);
-            v[3] = fmaf(wt[w], x0.w, v[3]);
-            v[4] = fmaf(wt[w], x1.x, v[4]);
-            v[5] = fmaf(wt[w], x1.y, v[5]);
-            v[6] = fmaf(wt[w], x1.z, v[6]);
-            v[7] = fmaf(wt[w], x1.w, v[7]);
+            const float mw = lds_ml[n][w][0][r];
+            wt[w] = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);
+            L = fmaf(wt[w], lds_ml[n][w][1][r], L);
         }
+        const float inv = L > 0.f ? 1.f / L : 0.f;
+        uint16_t* orow = a.out + ((size_t)(hq + n) * a.q_len + out_row) * D + dg * DPT;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] *= inv;
-        uint4 wv;
-        wv.x = (uint32_t)f32_to_bf16_rne(v[0]) | ((uint32_t)f32_to_bf16_rne(v[1]) << 16);
-        wv.y = (uint32_t)f32_to_bf16_rne(v[2]) | ((uint32_t)f32_to_bf16_rne(v[3]) << 16);
-        wv.z = (uint32_t)f32_to_bf16_rne(v[4]) | ((uint32_t)f32_to_bf16_rne(v[5]) << 16);
-        wv.w = (uint32_t)f32_to_bf16_rne(v[6]) | ((uint32_t)f32_to_bf16_rne(v[7]) << 16);
-        *reinterpret_cast<uint4*>(orow + d8) = wv;
+        for (int d8 = 0; d8 < DPT; d8 += 8) {
+            float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            const int g0 = (dg * DPT + d8) / 4;  // first of the two granules of these eight dims
+#pragma unroll
+            for (int w = 0; w < kRowWaves; ++w) {
+                const float4* wo = reinterpret_cast<const float4*>(&lds[w][0][0]) + r * GR;
+                const float4 x0 = wo[g0 ^ (r % GR)];
+                const float4 x1 = wo[(g0 + 1) ^ (r % GR)];
+                v[0] = fmaf(wt[w], x0.x, v[0]);
+                v[1] = fmaf(wt[w], x0.y, v[1]);
+                v[2] = fmaf(wt[w], x0.z, v[2]);
+                v[3] = fmaf(wt[w], x0.w, v[3]);
+                v[4] = fmaf(wt[w], x1.x, v[4]);
+                v[5] = fmaf(wt[w], x1.y, v[5]);
+                v[6] = fmaf(wt[w], x1.z, v[6]);
+                v[7] = fmaf(wt[w], x1.w, v[7]);
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] *= inv;
+            uint4 wv;
+            wv.x = (uint32_t)f32_to_bf16_rne(v[0]) | ((uint32_t)f32_to_bf16_rne(v[1]) << 16);
+            wv.y = (uint32_t)f32_to_bf16_rne(v[2]) | ((uint32_t)f32_to_bf16_rne(v[3]) << 16);
+            wv.z = (uint32_t)f32_to_bf16_rne(v[4]) | ((uint32_t)f32_to_bf16_rne(v[5]) << 16);
+            wv.w = (uint32_t)f32_to_bf16_rne(v[6]) | ((uint32_t)f32_to_bf16_rne(v[7]) << 16);
+            *reinterpret_cast<uint4*>(orow + d8) = wv;
+        }
+        if (dg == 0 && a.lse != nullptr)
+            a.lse[(size_t)(hq + n) * a.q_len + out_row] = L > 0.f ? (M + log2f(L)) * kLn2 : -INFINITY;
     }
-    if (dg == 0 && a.lse != nullptr)
-        a.lse[(size_t)hq * a.q_len + out_row] = L > 0.f ? (M + log2f(L)) * kLn2 : -INFINITY;
 }
 
 // Row-block kernel shape: 8 waves (two per SIMD: one wave's MFMAs run while the other waits on
 // LDS or loads), one K and one V tile each: 128 KiB of LDS at D = 128.
 constexpr int kRowWaves = 8;
 
-template <int D>
+template <int D, int HT>
 hipError_t launch_prefill_rows_t(const PrefillArgs& a, const Launch& l) {
-    const int n_rb = (a.q_len + kRows - 1) / kRows;
-    const int G = a.n_q_heads / a.n_kv_heads;
-    dim3 grid(a.n_kv_heads, G * n_rb);
+    const dim3 grid(a.n_kv_heads, a.n_q_heads / a.n_kv_heads / HT * ((a.q_len + kRows - 1) / kRows));
     if (a.block_table != nullptr)
-        return launch_kernel(prefill_rows_kernel<D, true, kRowWaves>, grid, dim3(kRowWaves * 64), l, a);
-    return launch_kernel(prefill_rows_kernel<D, false, kRowWaves>, grid, dim3(kRowWaves * 64), l, a);
+        return launch_kernel(prefill_rows_kernel<D, true, kRowWaves, HT>, grid, dim3(kRowWaves * 64), l, a);
+    return launch_kernel(prefill_rows_kernel<D, false, kRowWaves, HT>, grid, dim3(kRowWaves * 64), l, a);
 }
 
 // Merge of a row's KV segments.  Segment s holds keys [s*seg_len, (s+1)*seg_len); a row
@@ -1364,8 +1418,10 @@ hipError_t launch_prefill_combine(int head_dim, const PrefillArgs& a, const Laun
 
 hipError_t launch_prefill_rows(int head_dim, const PrefillArgs& a, const Launch& l) {
     if ((a.q_len + kRows - 1) / kRows * (a.n_q_heads / a.n_kv_heads) > 65535) return hipErrorInvalidValue;
-    if (head_dim == 128) return launch_prefill_rows_t<128>(a, l);
-    if (head_dim == 64) return launch_prefill_rows_t<64>(a, l);
+    if (a.rows_heads == 2)
+        return head_dim == 128 && a.n_q_heads / a.n_kv_heads % 2 == 0 ? launch_prefill_rows_t<128, 2>(a, l) : hipErrorInvalidValue;
+    if (head_dim == 128) return launch_prefill_rows_t<128, 1>(a, l);
+    if (head_dim == 64) return launch_prefill_rows_t<64, 1>(a, l);
     return hipErrorInvalidValue;
 }
 

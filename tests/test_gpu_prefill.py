@@ -539,6 +539,35 @@ def test_segment_workspace_stays_with_its_stream():
                 check_rows(o.cpu().numpy().view(np.uint16), None, ref, None)
 
 
+@pytest.mark.parametrize("hq,hkv,q_len,history,causal,paged", [
+    (32, 8, 257, 500, True, False), (32, 8, 512, 0, False, False), (32, 8, 385, 33, True, True),
+    (16, 8, 600, 301, True, False), (64, 4, 159, 64, True, True), (8, 2, 1056, 1500, True, False)])
+def test_row_blocks_of_two_heads(hq, hkv, q_len, history, causal, paged):
+    """Launches of more (row block, head) pairs than CUs take two heads per work-group: word for word the rows of
+    launches of few rows, which take one, and within the oracle's bound; the appended rows are in the cache."""
+    rng = np.random.default_rng(hq + hkv + q_len + history)
+    L = history + q_len
+    q, k, v = (bf16_normal(rng, (h, n, 128)) for h, n in ((hq, q_len), (hkv, L), (hkv, L)))
+    kw = dict(page_size=64) if paged else {}
+    with AttentionAccelerator(n_q_heads=hq, n_kv_heads=hkv, max_seq_len=L, max_q_len=q_len, **kw) as acc:
+        set_prefill_kernel(acc, "rows")
+        if paged:
+            acc.reserve(0, L)
+        if history:
+            acc.load_kv(k[:, :history], v[:, :history])
+        print(f"[two heads] {hq}/{hkv} {q_len} after {history}", flush=True)
+        out, lse = acc.prefill_chunk(q, q_pos_base=history, kv_len=L, k_rows=k[:, history:], v_rows=v[:, history:],
+                                     causal=causal, return_lse=True)
+        kr, vr = acc.read_kv(0, 0, L)
+        assert np.array_equal(kr, k) and np.array_equal(vr, v)
+        for at in range(0, q_len, 64):
+            o1, l1 = acc.prefill_chunk(q[:, at:at + 64], q_pos_base=history + at, kv_len=L, causal=causal, return_lse=True)
+            assert np.array_equal(out[:, at:at + 64], o1)
+            assert np.array_equal(lse[:, at:at + 64].view(np.uint32), l1.view(np.uint32))
+    ref, ref_lse = oracle_for(q, k, v, causal=causal, q_pos_base=history)
+    check_rows(out, lse, ref, ref_lse)
+
+
 @pytest.mark.parametrize("L", [1, 63, 64, 301, 512])
 def test_transaction_staging(L):
     """Q and the output share the context's pinned buffer, in up to four parts: a query submitted twice before the
