@@ -168,3 +168,26 @@ def test_kv260_mode_span_edges(L):
         out, want = run_both(q, k, v, causal=causal, qb=0, kb=0)
         mism = np.argwhere(out != want)
         assert mism.size == 0, f"{len(mism)} mismatching words, first at {tuple(mism[0])}"
+
+
+@pytest.mark.parametrize("kind,log2_scale", [("small", -100), ("mixed", -60), ("mixed", -24), ("mixed", -23)])
+@pytest.mark.parametrize("L,d", [(79, 128), (273, 64)])
+def test_kv260_mode_scaled_scores_that_wrap(kind, log2_scale, L, d):
+    """Words inside the native range under a scale that takes their scores below the normal range: the board's
+    exponent wraps where a native product becomes subnormal or zero."""
+    rng = np.random.default_rng(2600 + L + d)
+    q, k, v = (bf16_normal(rng, (h, L, d)) for h in (4, 2, 2))
+    if kind == "small":
+        q, k = bf16_normal(rng, q.shape, 2.0 ** -30), bf16_normal(rng, k.shape, 2.0 ** -30)
+    else:  # every row at an exponent of its own, from the lowest of the range to one
+        for t in (q, k):
+            t &= np.uint16(0x807F)
+            t |= (rng.integers(71, 128, t.shape[:2] + (1,)) << 7).astype(np.uint16)
+    with AttentionAccelerator(n_q_heads=4, n_kv_heads=2, head_dim=d, max_seq_len=L, scale=2.0 ** log2_scale,
+                              numerics="kv260") as acc:
+        for causal in (True, False):
+            print(f"[kv260] {kind} scale=2^{log2_scale} L={L} d={d} causal={causal}", flush=True)
+            out = acc.run_attention(q, k, v, causal=causal)
+            want, _, _ = rtl.attention(q, k, v, causal=causal, scale=acc.scale)
+            mism = np.argwhere(out != want)
+            assert mism.size == 0, f"{len(mism)} mismatching words, first at {tuple(mism[0])}"
