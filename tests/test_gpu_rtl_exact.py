@@ -191,3 +191,30 @@ def test_kv260_mode_scaled_scores_that_wrap(kind, log2_scale, L, d):
             want, _, _ = rtl.attention(q, k, v, causal=causal, scale=acc.scale)
             mism = np.argwhere(out != want)
             assert mism.size == 0, f"{len(mism)} mismatching words, first at {tuple(mism[0])}"
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_kv260_mode_infinite_o_word_forgotten(d):
+    """An O word that wraps to exponent 255 (each sub-block's max rises by the x whose table value is 2^-4, V zero
+    behind a first 2^-56) and then a correction of zero: the board's product is zero, not NaN."""
+    x = -float.fromhex("-0x1.62e47p1")
+    assert rtl.exp_lookup(np.float32([-x]).view(np.uint32))[0] == 0x3D800000
+    scores = np.array([x * (j - 9) for j in range(19)] + [40.0], np.float32).repeat(16)
+    L = scores.size
+    q, k, v = np.zeros((4, L, d), np.uint16), np.zeros((2, L, d), np.uint16), np.zeros((2, L, d), np.uint16)
+    q[:, :, :3] = 0x3F80
+    rest = scores.copy()
+    for i in range(3):  # the score in three exact bf16 pieces
+        k[:, :, i] = rest.view(np.uint32) >> 16
+        rest = rest - (rest.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+    assert not rest.any()
+    v[:, 0, :] = (71 << 7) | (np.arange(d) % 2 << 15)
+    v[:, -16:, :] = bf16_normal(np.random.default_rng(2700 + d), (2, 16, d))
+    with AttentionAccelerator(n_q_heads=4, n_kv_heads=2, head_dim=d, max_seq_len=L, scale=1.0, numerics="kv260") as acc:
+        for causal in (True, False):
+            print(f"[kv260] infinite O d={d} causal={causal}", flush=True)
+            out = acc.run_attention(q, k, v, causal=causal)
+            want, _, _ = rtl.attention(q, k, v, causal=causal, scale=1.0)
+            assert np.any(want[:, 18 * 16:19 * 16] & 0x7F80 == 0x7F80) == causal and not np.any(want[:, -1] & 0x7F80 == 0x7F80)
+            mism = np.argwhere(out != want)
+            assert mism.size == 0, f"{len(mism)} mismatching words, first at {tuple(mism[0])}"
