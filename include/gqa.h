@@ -65,10 +65,13 @@ extern "C" {
 /* Tunables for gqa_set_option. */
 #define GQA_OPT_DECODE_CHUNK 1 /* keys per split-KV work-group (a multiple of 64 giving at most max(l_cap / 256,
                                   the automatic plan's) splits; a last split of <= chunk/4 keys joins the one
-                                  before it; 0 = auto: about 8 waves per CU, whole 16-key rounds per wave).
+                                  before it; 0 = auto: about 8 waves per CU, whole 16-key rounds per wave, or
+                                  in 64-key steps about 112 work-groups per 256 CUs where K/V of at most
+                                  16 MiB would need a merge launch and merge in the decode launch that way).
                                   The automatic plan does not split a (sequence, kv head) whose K/V take
-                                  at most 128 KiB (256 KiB from 32 of them on).  Work-groups have 8 waves, or 4 when the 8-wave plan
-                                  has at most 8 work-groups (the automatic chunk is then planned for 4) */
+                                  at most 128 KiB (256 KiB from 32 of them on).  Work-groups have 8 waves, or
+                                  4 when the 8-wave plan has at most 8 work-groups (the automatic chunk is
+                                  then planned for 4) */
 #define GQA_OPT_PROFILE      2 /* 1 = time every kernel launch with a HIP event pair bound to the launch
                                   (hipExtLaunchKernel; restarts the record).  Binding adds no GPU work
                                   between launches, but each timed launch costs the host several us,
@@ -106,10 +109,11 @@ extern "C" {
  * finish merges the others' partials inside the decode launch (agent-scope atomics and a per-unit
  * arrival counter; one launch per step).  LAUNCH: a second, log-sum-exp merge launch.  AUTO (default):
  * FUSED while the split grid (sequences x kv heads x splits) is at most half the GPU's CU count and a
- * sequence has at most 32 splits -- every split ends with an L2 write-back of its XCD and an increment
- * of its sequence's counter, which saves the launch for short steps but slows the streaming of larger
- * grids more than a launch costs -- else LAUNCH.  An automatic plan of the shortest splits (one round
- * of every wave) that would need the merge launch takes splits twice as long where that lets AUTO fuse.
+ * sequence has at most 16 splits (32 in the automatic plan's 64-key steps) -- every split ends with an L2
+ * write-back of its XCD and an increment of its sequence's counter, which saves the launch for short steps
+ * but slows the streaming of larger grids more than a launch costs -- else LAUNCH.  An automatic plan of the
+ * shortest splits (one round of every wave) that would need the merge launch takes splits twice as long
+ * where that lets AUTO fuse.
  * Both fold the splits in the same order (the same output words). */
 #define GQA_DECODE_MERGE_AUTO   0
 #define GQA_DECODE_MERGE_LAUNCH 1

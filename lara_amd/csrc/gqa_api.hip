@@ -205,8 +205,9 @@ int plan_splits(int batch, int n_kv_heads, int n_cu, int waves) {
 // per unit: 4.2 us of kernel in one split per unit against 4.8 us in four splits merged in-launch).
 // With kUnsplitUnits units and more the GPU has work enough without splits up to twice that (us a step over three
 // streams / on one, split against unsplit: 8 sequences of 300 keys, 32/8 heads of 128, 8.1 / 9.3 against 4.4 /
-// 6.0; 16 of 500 8.7 / 11.0 against 5.8 / 9.3; 40 of 600, 8/2 heads of 64, 8.1 / 9.1 against 4.4 / 6.4; but one of 500, 8
-// units, 4.3 / 7.0 against 4.4 / 9.1).
+// 6.0; 16 of 500 8.7 / 11.0 against 5.8 / 9.3; 40 of 600, 8/2 heads of 64, 8.1 / 9.1 against 4.4 / 6.4; at 32 units, 16
+// of 700, 32/2 heads of 64, 5.2 / 9.4 against 4.6 / 7.5, 4 of 1000, 32/8 heads of 64, 4.7 / 7.8 either way; but one of
+// 500, 8 units, 4.3 / 7.0 against 4.4 / 9.1).
 constexpr int64_t kDecodeSplitMinBytes = 128 << 10;
 constexpr int kUnsplitUnits = 32;
 
@@ -227,12 +228,12 @@ int plan_chunk(int batch, int n_kv_heads, int group, int n_cu, int max_len, int 
 // sequence's arrival counter, and the last one with an acquire (an L2 invalidate): that saves the
 // merge launch where the step is a short latency chain, but the L2 maintenance of many work-groups
 // slows the streaming of the others.  AUTO fuses up to kFusedMergeSplits splits per sequence while
-// the split grid fills at most half the CUs (16 of them until the plans below bounded the grid; measured, kernel time per step, fused vs launch: 4
+// the split grid fills at most half the CUs (measured, kernel time per step, fused vs launch: 4
 // work-groups (2 splits of 128 keys) 5.1 vs 8.1 us, 64 work-groups (8 splits of 512) 9.4 vs 11.7 us,
 // 32 q / 8 kv heads, one sequence of 2049 keys: 128 work-groups (16 splits of 128) 7.5 vs 8.6 us;
 // 256 work-groups: 8 splits of 16384 keys 314.1 vs 311.5 us, 4 of 8192 161 vs 160 us, 2 of 4096
 // 83-86 vs 81-82 us, 2 of 512 16.7 vs 16.1 us; 32 splits of 128 keys 9.4 vs 8.8 us).
-constexpr int kFusedMergeSplits = 32;
+constexpr int kFusedMergeSplits = 16;
 
 bool fuse_merge(int option, int units, int max_splits, int n_cu) {
     if (max_splits <= 1 || option == GQA_DECODE_MERGE_LAUNCH) return false;
@@ -253,58 +254,60 @@ bool fuse_merge(int option, int units, int max_splits, int n_cu) {
 // of 2049 keys, 8 fused splits of 256 8.50 against 16 of 128 and a launch 9.00).
 constexpr int64_t kSmallDecodeGrid = 8;
 
-// Two more ranges of the automatic plan, in splits of whole 64-key steps (us a step over three streams / on one,
-// before against after):
-//  - K/V of at most kFusedPlanBytes over at most kFusedPlanUnits units: about kFusedPlanGrid work-groups merged
-//    in-launch.  A grid that fills the CUs pays a merge launch, or an L2 write-back per work-group, for a
-//    stream of a few us: one sequence of 8000 keys, 8/2 heads of 64, 7.9 / 9.4 against 4.4 / 7.3 (62
-//    work-groups); 10 of 2000 8.1 / 9.1 against 5.2 / 8.0; 4 of 1000, 32/8 heads of 128, 7.1 / 9.1 against 6.0 / 9.0; 7
-//    of up to 3000, 32/2 heads of 64, 8.0 / 10.8 against 5.5 / 10.9.
-//  - up to kStreamPlanBytes over 8 units to kFusedPlanUnits, in splits of three rounds a wave and more:
-//    kStreamPlanGrid work-groups merged by a launch, which leaves room for the merge of the launch before: one of
-//    16000 keys, 32/8 heads of 128, 11.9 / 15.7 against 11.7 / 15.0; of 30000 20.0 / 23.7 against 18.9 / 23.1; of
-//    20000, 64/8 heads, 15.1 / 19.2 against 14.7 / 18.7; 4 of 4000 13.1 / 15.0 against 11.7 / 15.3.  (Shorter splits
-//    gained nothing; above, 530 MB: 79.2 / 85.4 on 256 work-groups, 75.9 / 97.6 on 128, every CU streams.)
-constexpr int64_t kFusedPlanBytes = 16 << 20, kStreamPlanBytes = 128 << 20;
-constexpr int kFusedPlanUnits = 32;
-constexpr double kFusedPlanGrid = 112.0 / 256, kStreamPlanGrid = 208.0 / 256;  // of the CUs
+// Where that plan would still need the merge launch, K/V of at most kFusedPlanBytes over at most kFusedPlanUnits
+// units take about kFusedPlanGrid work-groups of 64-key steps instead, merged in-launch in up to
+// kFusedPlanSplits splits.  A grid that fills the CUs pays a second launch for a stream of a few us, and beside
+// other streams its work-groups too (us a step over three streams / on one, launch against in-launch: one
+// sequence of 8000 keys, 8/2 heads of 64, 7.2 / 8.6 against 4.5 / 7.4; 3 of 1500, 32/8 heads of 64, 7.1 / 8.2
+// against 4.8 / 8.0; one of 3000 in a cache of 8192 rows, 32/2 heads of 64, 6.8 / 8.6 against 4.5 / 9.0).
+// In-launch splits longer than kFusedPlanKeys lose more on one stream than the launch costs (8 sequences of 4000,
+// 8/2 heads of 64, 576 keys 9.1 against 8.3 by a launch; one of 6000, 32/8 heads, 448 keys 8.2 against 8.1).
+// Groups above 8 take longer per key and merge: up to kFusedPlanKeysWide keys they still save other streams more
+// (7 of 200 .. 3000, 32/2 heads of 64, 7.1 / 10.3 against 5.9 / 11.1), beyond not (8 of 4096 7.5 / 9.9 against 7.9 / 11.5).
+// (The byte bound ends it before the keys do at D 128 alone.)  A plan that
+// merges in-launch as it is stays: its shorter splits are the better ones for sequences that end well before the
+// capacity (one of 1000 keys in 4096 rows, 64/8 heads of 128: 9.7 in splits of 256, 10.1 of 320; one of 300 there,
+// 32/2 heads of 64: 5.7 in splits of 256, 8.0 of 128).  So does a grid that needs a merge launch at any size: 208
+// work-groups instead of 256 to 264 gained at full caches (3 of 8000, 64/8 heads, 25.7 -> 21.0 on one stream) but lost as
+// much at a quarter of the capacity (3 of 2500 in 10000 rows 16.2 -> 20.7).
+constexpr int64_t kFusedPlanBytes = 16 << 20;
+constexpr int kFusedPlanUnits = 32, kFusedPlanSplits = 32;
+constexpr int kFusedPlanKeys = 448, kFusedPlanKeysWide = 384;  // (wide: groups above 8)
+constexpr double kFusedPlanGrid = 112.0 / 256;                 // of the CUs
 
 struct DecodeShape {
     int chunk;
     int max_splits;
     int waves;
+    bool fused;  // merged in-launch
 };
 
 DecodeShape plan_decode_shape(int batch, int n_kv_heads, int group, int head_dim, int n_cu, int max_len,
                               int chunk_opt, int merge_option) {
     const int64_t units = (int64_t)batch * n_kv_heads;
+    auto in_chunks = [&](int chunk, int waves) {
+        const int splits = decode_split_count(max_len, chunk);
+        return DecodeShape{chunk, splits, waves, fuse_merge(merge_option, (int)units, splits, n_cu)};
+    };
     auto shape = [&](int waves) {
-        const int chunk =
-            chunk_opt > 0 ? chunk_opt : plan_chunk(batch, n_kv_heads, group, n_cu, max_len, waves, head_dim);
-        return DecodeShape{chunk, decode_split_count(max_len, chunk), waves};
+        return in_chunks(chunk_opt > 0 ? chunk_opt : plan_chunk(batch, n_kv_heads, group, n_cu, max_len, waves, head_dim),
+                         waves);
     };
     const DecodeShape big = shape(kDecodeWaves);
     if (units * big.max_splits <= kSmallDecodeGrid) return shape(kDecodeWavesSmall);
-    const int64_t bytes = units * max_len * head_dim * 2 * 2;
-    if (chunk_opt <= 0 && merge_option == GQA_DECODE_MERGE_AUTO && big.max_splits > 1 && units <= kFusedPlanUnits &&
-        bytes <= kStreamPlanBytes) {
-        const bool fused = bytes <= kFusedPlanBytes;
-        const int grid = (int)((fused ? kFusedPlanGrid : kStreamPlanGrid) * n_cu);
-        const int splits = std::max(1, std::min(fused ? kFusedMergeSplits : INT_MAX, grid / (int)units));
-        const int shortest = kDecodeWaves * decode_round_keys(group);
-        const int even = ((max_len + splits - 1) / splits + kChunkOptionQuantum - 1) / kChunkOptionQuantum * kChunkOptionQuantum;
-        const DecodeShape s{std::max(shortest, even), decode_split_count(max_len, std::max(shortest, even)), kDecodeWaves};
-        if (fused ? s.max_splits > 1 && fuse_merge(merge_option, (int)units, s.max_splits, n_cu) : units >= 8 && s.chunk >= 3 * shortest)
-            return s;
+    if (chunk_opt > 0 || merge_option != GQA_DECODE_MERGE_AUTO || big.max_splits <= 1 || big.fused) return big;
+    const int shortest = kDecodeWaves * decode_round_keys(group);
+    if (big.chunk == shortest) {
+        const DecodeShape twice = in_chunks(2 * shortest, kDecodeWaves);
+        if (twice.fused) return twice;
     }
-    if (chunk_opt <= 0 && merge_option == GQA_DECODE_MERGE_AUTO && big.max_splits > 1 &&
-        big.chunk == kDecodeWaves * decode_round_keys(group) &&
-        !fuse_merge(merge_option, (int)units, big.max_splits, n_cu)) {
-        const int chunk = 2 * big.chunk;
-        const DecodeShape twice{chunk, decode_split_count(max_len, chunk), kDecodeWaves};
-        if (fuse_merge(merge_option, (int)units, twice.max_splits, n_cu)) return twice;
-    }
-    return big;
+    if (units > kFusedPlanUnits || units * max_len * head_dim * 2 * 2 > kFusedPlanBytes) return big;
+    const int splits = std::max(1, std::min(kFusedPlanSplits, (int)(kFusedPlanGrid * n_cu) / (int)units));
+    const int even = (max_len + splits - 1) / splits;
+    DecodeShape s = in_chunks(std::max(shortest, (even + kChunkOptionQuantum - 1) / kChunkOptionQuantum * kChunkOptionQuantum),
+                              kDecodeWaves);
+    s.fused = s.max_splits > 1 && s.max_splits <= kFusedPlanSplits && 2 * units * s.max_splits <= n_cu;
+    return s.fused && s.chunk <= (group > 8 ? kFusedPlanKeysWide : kFusedPlanKeys) ? s : big;
 }
 
 constexpr int kProfileLaunches = 512;  // event pairs kept per timer slot
@@ -384,8 +387,7 @@ int plan_decode(gqa_ctx* c, const void* q, const int32_t* lens, const void* k_ne
     a.longest_first = c->cfg.batch > 1;
     a.cached = decode_cached_loads((int64_t)c->cfg.batch * c->cfg.n_kv_heads, max_len, c->cfg.head_dim) ? 1 : 0;
     a.waves = shape.waves;
-    a.arrivals = fuse_merge(c->decode_merge, c->cfg.batch * c->cfg.n_kv_heads, max_splits, c->n_cu) ? c->arrivals
-                                                                                                      : nullptr;
+    a.arrivals = shape.fused ? c->arrivals : nullptr;
     *combine = max_splits > 1 && a.arrivals == nullptr;
     a.ticket = (c->cfg.batch > 1 && max_splits == 1) ? c->arrivals + (size_t)c->cfg.batch * c->cfg.n_kv_heads : nullptr;
     return GQA_OK;
@@ -1687,9 +1689,7 @@ int gqa_decode_append_noalloc(const gqa_config* cfg, void* k_cache, void* v_cach
     // The same merge as the context entry point's default (GQA_DECODE_MERGE_AUTO), when the counters
     // cover the units.
     const int units = k.batch * k.n_kv_heads;
-    a.arrivals = units <= kNoAllocCounters && fuse_merge(GQA_DECODE_MERGE_AUTO, units, max_splits, dev->n_cu)
-                     ? dev->arrivals
-                     : nullptr;
+    a.arrivals = units <= kNoAllocCounters && shape.fused ? dev->arrivals : nullptr;
     Launch l;
     l.stream = (hipStream_t)stream;
     HIP_TRY(launch_decode(k.head_dim, group, a, l));

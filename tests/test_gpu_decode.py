@@ -406,8 +406,8 @@ def test_decode_auto_plan_merges_small_grids_in_launch(B, hq, hkv, d, L, twice):
                                                  (1, 32, 8, 128, 16001, 2), (1, 64, 8, 128, 9973, 2), (3, 32, 8, 128, 5000, 2)])
 def test_decode_auto_plan_ranges(B, hq, hkv, d, L, merges):
     """The automatic plan's ranges: small K/V in about 112 work-groups merged in-launch or, from 32 (sequence, kv
-    head) units on, unsplit; larger ones in about 208 merged by a launch; ragged lengths with splits in 64-key
-    steps, each step against the oracle, twice (the arrival counters reset)."""
+    head) units on, unsplit; larger ones merged by a launch; ragged lengths with splits in 64-key steps, each step
+    against the oracle, twice (the arrival counters reset)."""
     torch = pytest.importorskip("torch")
     rng = np.random.default_rng(900 + B * 10 + d + L)
     lens = np.full(B, L, np.int32)
@@ -424,3 +424,22 @@ def test_decode_auto_plan_ranges(B, hq, hkv, d, L, merges):
             check_decode(out, lse, q, kc, vc, lens, None)
         if torch.cuda.get_device_properties(0).multi_processor_count == 256:
             assert _merge_launches(eng) == (merges, 2)
+
+
+@pytest.mark.parametrize("B,hq,hkv,d,L", [(4, 32, 2, 64, 8000), (16, 8, 2, 64, 4096), (1, 8, 2, 64, 24000), (14, 32, 2, 64, 2000)])
+def test_decode_auto_plan_keeps_the_merge_launch(B, hq, hkv, d, L):
+    """Small K/V whose in-launch splits would be longer than the automatic plan takes (448 keys, 384 in groups above
+    8) are cut for the whole GPU and merged by a launch; ragged lengths, each step against the oracle."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(950 + B * 10 + d + L)
+    lens = rng.integers(1, L + 1, B).astype(np.int32)
+    lens[0] = L
+    print(f"[plan] B={B} hq={hq} hkv={hkv} d={d} L={L}", flush=True)
+    with make_engine(B, hq, hkv, d, L) as eng:
+        kc, vc = fill_cache(eng, rng, B, hkv, d, lens, lcap=L)
+        _lib.check(eng._lib.gqa_set_option(eng._ctx, _lib.GQA_OPT_PROFILE, 1), "profile")
+        q = bf16_normal(rng, (B, hq, d))
+        out, lse = eng.decode_step(q, lens, return_lse=True)
+        check_decode(out, lse, q, kc, vc, lens, None)
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            assert _merge_launches(eng) == (1, 1)
