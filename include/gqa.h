@@ -97,9 +97,11 @@ extern "C" {
  * round, which longest-first dispatch cannot balance); else, when the SHARED grid without segments has
  * fewer work-groups than the GPU has CUs, ROWS or, where its estimate is the shorter (few rows after
  * thousands of earlier keys), SHARED in one or more KV segments (several only on the first stream that
- * needs the segments' workspace, and not under a capture); else SHARED -- paired when that grid is exactly
+ * needs the segments' workspace, and not under a capture or in caches of at most 1024 rows); else SHARED -- paired when that grid is exactly
  * one work-group per CU (for instance a causal 2048-row chunk after earlier keys at 32q/8kv on 256
- * CUs), unpaired when larger.  gqa_last_prefill_plan reports the decomposition a launch took. */
+ * CUs), unpaired when larger.  gqa_last_prefill_plan reports the decomposition a launch took.
+ * Launches in several segments under a forced decomposition or segment target share a workspace of their own:
+ * the caller orders them among each other (streams, replayed graphs); AUTO's may be in flight beside them. */
 #define GQA_PREFILL_KERNEL_AUTO   0
 #define GQA_PREFILL_KERNEL_SHARED 1
 #define GQA_PREFILL_KERNEL_ROWS   2

@@ -21,6 +21,8 @@ namespace {
 constexpr int kChunkOptionQuantum = 64;  // GQA_OPT_DECODE_CHUNK: a multiple of every decode round size
 constexpr int kMinSplitCap = 256;        // the split workspace holds at least l_cap / this splits
 constexpr int kMaxPrefillSegs = 32;
+constexpr int kAutoSegmentKeys = 1024;   // caches of at most this many rows have no workspace for automatic segments,
+                                         // which save time on longer spans only (up to 32 kv heads)
 constexpr int32_t kMaxRows = 1 << 30;  // max_seq_len / max_q_len limit: row counts rounded up stay in int32
 constexpr double kRopeBase = 10000.0;  // theta_p = 10000^(-2p/D): hw/data/rope_theta.hex for D = 128
 constexpr int kDecodeWavesPerCu = 8;  // split planner target; one split per (sequence, kv head) once that fills the GPU
@@ -74,11 +76,12 @@ struct gqa_ctx {
                                   // of one-split launches (all zero between launches)
     int decode_merge = GQA_DECODE_MERGE_AUTO;
     int prefill_kernel = GQA_PREFILL_KERNEL_AUTO;
-    float* pre_ws = nullptr;     // prefill KV-segment partials (O, then (m, l))
+    float* pre_ws = nullptr;     // prefill KV-segment partials (O, then (m, l)) of launches with a forced decomposition
+    float* auto_ws = nullptr;    // the same of the automatic plan's, which may be in flight beside those
     uint16_t* zero_row = nullptr;  // one zero K/V row: the prefill source of rows past kv_len
-    size_t pre_ws_floats = 0;
-    bool pre_ws_bound = false;     // the stream whose automatically segmented launches use it
-    hipStream_t pre_ws_stream = nullptr;
+    size_t pre_ws_floats = 0, auto_ws_floats = 0;
+    bool auto_ws_bound = false;    // the stream whose automatically segmented launches use it
+    hipStream_t auto_ws_stream = nullptr;
     uint16_t* q_dev = nullptr;   // staging: max(B*H_q*D, H_q*max_q_len*D) words
     uint16_t* o_dev = nullptr;   // same size as q_dev
     float* lse_dev = nullptr;    // max(B*H_q, H_q*max_q_len)
@@ -554,11 +557,11 @@ int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_p
     if (segs > 1) {
         // The partials' workspace belongs to the first stream that needs it: launches on other streams and
         // captured ones (a graph may replay beside anything) may overlap with that stream's and use none.
-        if (!c->pre_ws_bound && !stream_capturing(s)) {
-            c->pre_ws_bound = true;
-            c->pre_ws_stream = s;
+        if (!c->auto_ws_bound && !stream_capturing(s)) {
+            c->auto_ws_bound = true;
+            c->auto_ws_stream = s;
         }
-        if (!c->pre_ws_bound || c->pre_ws_stream != s || stream_capturing(s)) segs = segments(1);
+        if (!c->auto_ws_bound || c->auto_ws_stream != s || stream_capturing(s)) segs = segments(1);
     }
     // A forced PAIRED decomposition plans one KV segment (pairs exist only in one-segment launches);
     // launches it cannot pair (not causal, group != 4, one row block) plan as SHARED.
@@ -567,7 +570,9 @@ int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_p
                        : segs > 0                 ? segs * shared_wgs
                                                   : c->n_cu;
     PrefillPlan plan = plan_prefill(q_len, kv_span, c->group, c->cfg.n_kv_heads, target, kMaxPrefillSegs);
-    const bool fits = prefill_workspace_floats(plan, q_len, c->cfg.n_q_heads, c->cfg.head_dim) <= c->pre_ws_floats;
+    float* const ws = plan_auto ? c->auto_ws : c->pre_ws;
+    const bool fits = prefill_workspace_floats(plan, q_len, c->cfg.n_q_heads, c->cfg.head_dim) <=
+                      (plan_auto ? c->auto_ws_floats : c->pre_ws_floats);
     if (!fits) plan = plan_prefill(q_len, kv_span, c->group, c->cfg.n_kv_heads, 1, 1);  // one segment
     const bool rows = c->prefill_kernel == GQA_PREFILL_KERNEL_ROWS || (plan_auto && (segs == 0 || !fits));
     PrefillArgs a{};
@@ -595,8 +600,8 @@ int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_p
     a.seg_len = plan.seg_len;
     a.n_segs = plan.n_segs;
     a.zero_row = c->zero_row;
-    a.part_o = c->pre_ws;
-    a.part_ml = c->pre_ws + (size_t)plan.n_segs * c->cfg.n_q_heads * q_len * c->cfg.head_dim;
+    a.part_o = ws;
+    a.part_ml = ws + (size_t)plan.n_segs * c->cfg.n_q_heads * q_len * c->cfg.head_dim;
     if (rows) {
         a.rows_heads = rows_two_heads(q_len, kv_span, causal != 0, c->group, c->cfg.n_kv_heads, c->cfg.head_dim, c->n_cu) ? 2 : 1;
         HIP_TRY(launch_prefill_rows(c->cfg.head_dim, a, timed(c, GQA_TIMER_PREFILL, s)));
@@ -1027,6 +1032,8 @@ int create_ctx(const gqa_config* cfg, int32_t page_size, int32_t n_pages, int32_
     if (prefill_supported(k.head_dim, group)) {
         c->pre_ws_floats = prefill_workspace_need(c, c->n_cu);
         if (c->pre_ws_floats > 0) alloc((void**)&c->pre_ws, c->pre_ws_floats * sizeof(float));
+        if (k.max_seq_len > kAutoSegmentKeys) c->auto_ws_floats = c->pre_ws_floats;
+        if (c->auto_ws_floats > 0) alloc((void**)&c->auto_ws, c->auto_ws_floats * sizeof(float));
     }
     alloc((void**)&c->q_dev, c->stage_words * 2);
     alloc((void**)&c->o_dev, c->stage_words * 2);
@@ -1223,6 +1230,7 @@ int gqa_destroy(gqa_ctx* c) {
     (void)hipFree(c->part_ml);
     (void)hipFree(c->arrivals);
     (void)hipFree(c->pre_ws);
+    (void)hipFree(c->auto_ws);
     (void)hipFree(c->zero_row);
     (void)hipFree(c->q_dev);
     (void)hipFree(c->o_dev);

@@ -600,3 +600,56 @@ def test_transaction_staging(L):
     for out, qq in ((first, q), (other, q2)):
         ref, _ = oracle_for(qq, k, v, causal=True)
         check_rows(out, None, ref, None)
+
+
+@pytest.mark.parametrize("forced", ["kernel", "work-groups"])
+def test_forced_segments_beside_automatic_ones(forced):
+    """A segmented launch under a forced decomposition, captured and replayed on a stream of its own, beside an
+    automatic segmented one: their partials do not share memory."""
+    torch = pytest.importorskip("torch")
+    import ctypes
+
+    from lara_amd import _lib
+
+    rng = np.random.default_rng(5300)
+    hq, hkv, d, q_len, kv_len = 32, 8, 128, 16, 9000
+    k, v = bf16_normal(rng, (hkv, kv_len, d)), bf16_normal(rng, (hkv, kv_len, d))
+    qs = [bf16_normal(rng, (hq, q_len, d)) for _ in range(2)]
+    refs = [oracle_for(q, k, v, causal=True, q_pos_base=kv_len - q_len)[0] for q in qs]
+    with AttentionAccelerator(max_seq_len=kv_len, max_q_len=64) as acc:
+        acc.load_kv(k, v)
+        q_dev = [torch.from_numpy(q.view(np.int16)).cuda() for q in qs]
+        o_dev = [torch.zeros_like(q) for q in q_dev]
+        torch.cuda.synchronize()
+
+        def launch(i, stream):
+            _lib.check(acc._lib.gqa_prefill_device(acc._ctx, 0, ctypes.c_void_p(q_dev[i].data_ptr()), q_len,
+                                                   kv_len - q_len, kv_len, 0, 1, ctypes.c_void_p(o_dev[i].data_ptr()),
+                                                   None, ctypes.c_void_p(stream)), "prefill")
+            return acc.last_prefill_plan()
+
+        def force(on):
+            if forced == "kernel":
+                set_prefill_kernel(acc, "shared" if on else "auto")
+            else:
+                _lib.check(acc._lib.gqa_set_option(acc._ctx, _lib.GQA_OPT_PREFILL_WGS, 200 if on else 0), "segments")
+
+        s0, s1 = torch.cuda.Stream(), torch.cuda.Stream()
+        graph = torch.cuda.CUDAGraph()
+        force(True)
+        with torch.cuda.graph(graph, stream=s1):
+            kernel, segs = launch(0, s1.cuda_stream)
+            assert kernel == "shared" and segs > 1
+        force(False)
+        for rep in range(4):
+            print(f"[segments] forced {forced} beside automatic, {rep}", flush=True)
+            for o in o_dev:
+                o.zero_()
+            torch.cuda.synchronize()
+            for _ in range(8):
+                with torch.cuda.stream(s1):
+                    graph.replay()
+                assert launch(1, s0.cuda_stream)[1] > 1
+            torch.cuda.synchronize()
+            for o, ref in zip(o_dev, refs):
+                check_rows(o.cpu().numpy().view(np.uint16), None, ref, None)
