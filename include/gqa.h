@@ -96,10 +96,11 @@ extern "C" {
  * keys before its own and whose SHARED grid holds half to one work-group per CU (a single dispatch
  * round, which longest-first dispatch cannot balance); else, when the SHARED grid without segments has
  * fewer work-groups than the GPU has CUs, ROWS or, where its estimate is the shorter (few rows after
- * thousands of earlier keys), SHARED in one or more KV segments (several only on the first stream that
- * needs the segments' workspace, and not under a capture or in caches of at most 1024 rows); else SHARED -- paired when that grid is exactly
- * one work-group per CU (for instance a causal 2048-row chunk after earlier keys at 32q/8kv on 256
- * CUs), unpaired when larger.  gqa_last_prefill_plan reports the decomposition a launch took.
+ * thousands of earlier keys), SHARED in one or more KV segments (several not under a capture, not in caches
+ * of at most 1024 rows, and on one stream at a time: the first that needs the segments' workspace, then one
+ * that asks for it a second time without a launch of that stream in between); else SHARED -- paired when
+ * that grid is exactly one work-group per CU (for instance a causal 2048-row chunk after earlier keys at
+ * 32q/8kv on 256 CUs), unpaired when larger.  gqa_last_prefill_plan reports the decomposition a launch took.
  * Launches in several segments under a forced decomposition or segment target share a workspace of their own:
  * the caller orders them among each other (streams, replayed graphs); AUTO's may be in flight beside them. */
 #define GQA_PREFILL_KERNEL_AUTO   0

@@ -80,8 +80,11 @@ struct gqa_ctx {
     float* auto_ws = nullptr;    // the same of the automatic plan's, which may be in flight beside those
     uint16_t* zero_row = nullptr;  // one zero K/V row: the prefill source of rows past kv_len
     size_t pre_ws_floats = 0, auto_ws_floats = 0;
-    bool auto_ws_bound = false;    // the stream whose automatically segmented launches use it
-    hipStream_t auto_ws_stream = nullptr;
+    bool auto_ws_bound = false;    // the stream whose automatically segmented launches use it, and another that
+    hipStream_t auto_ws_stream = nullptr;  // has asked for it since (take_auto_ws); only compared: it may be gone
+    bool auto_ws_asked = false;
+    hipStream_t auto_ws_asker = nullptr;
+    hipEvent_t ev_auto_ws = nullptr;       // the last launch that used it has ended
     uint16_t* q_dev = nullptr;   // staging: max(B*H_q*D, H_q*max_q_len*D) words
     uint16_t* o_dev = nullptr;   // same size as q_dev
     float* lse_dev = nullptr;    // max(B*H_q, H_q*max_q_len)
@@ -492,6 +495,34 @@ int plan_shared_segments(int q_len, int kv_span, bool causal, int group, int n_k
     return best;
 }
 
+// Whether a launch on s may use the automatic plan's partials.  One stream at a time has them: the first that
+// wants them, then any that asks for the second time without a launch of the owner in between (a program that has
+// moved its long prompts to another stream), while streams that take turns stay with one owner and plan without.
+// Captured launches never do: a graph may replay beside anything.  A caller's handle does not name a stream for
+// good (a destroyed one's can come back, hipStreamPerThread is one for every thread), so each launch on one marks
+// its end and waits for the mark before it (us a launch on one stream, 8 rows after 4000 keys: 14.3 -> 15.5; the
+// row-block kernel 22).  The context's own stream, which callers that pass none take, is marked only where another
+// takes over.
+bool take_auto_ws(gqa_ctx* c, hipStream_t s) {
+    if (stream_capturing(s)) return false;
+    const bool own = c->auto_ws_stream == c->stream;
+    if (c->auto_ws_bound && c->auto_ws_stream != s && !(c->auto_ws_asked && c->auto_ws_asker == s)) {
+        c->auto_ws_asked = true;
+        c->auto_ws_asker = s;
+        return false;
+    }
+    if (c->auto_ws_bound && !(own && s == c->stream) &&
+        ((own && hipEventRecord(c->ev_auto_ws, c->stream) != hipSuccess) ||
+         hipStreamWaitEvent(s, c->ev_auto_ws, 0) != hipSuccess)) {
+        (void)hipGetLastError();
+        return false;
+    }
+    c->auto_ws_bound = true;
+    c->auto_ws_stream = s;
+    c->auto_ws_asked = false;
+    return true;
+}
+
 int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_pos_base, int32_t kv_len,
                 int32_t kv_pos_base, int32_t causal, void* o, float* lse, hipStream_t s,
                 const void* k_new = nullptr, const void* v_new = nullptr, int32_t n_new = 0) {
@@ -553,28 +584,25 @@ int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_p
         return plan_shared_segments(q_len, kv_span, causal != 0, c->group, c->cfg.n_kv_heads, c->cfg.head_dim, c->n_cu,
                                     max_segs);
     };
+    auto plan_for = [&](int target_wgs, int max_segs) {
+        return plan_prefill(q_len, kv_span, c->group, c->cfg.n_kv_heads, target_wgs, max_segs);
+    };
     int segs = plan_auto ? segments(kMaxPrefillSegs) : 0;
-    if (segs > 1) {
-        // The partials' workspace belongs to the first stream that needs it: launches on other streams and
-        // captured ones (a graph may replay beside anything) may overlap with that stream's and use none.
-        if (!c->auto_ws_bound && !stream_capturing(s)) {
-            c->auto_ws_bound = true;
-            c->auto_ws_stream = s;
-        }
-        if (!c->auto_ws_bound || c->auto_ws_stream != s || stream_capturing(s)) segs = segments(1);
-    }
+    if (segs > 1 && (prefill_workspace_floats(plan_for(segs * shared_wgs, kMaxPrefillSegs), q_len, c->cfg.n_q_heads,
+                                              c->cfg.head_dim) > c->auto_ws_floats ||
+                     !take_auto_ws(c, s)))
+        segs = segments(1);
     // A forced PAIRED decomposition plans one KV segment (pairs exist only in one-segment launches);
     // launches it cannot pair (not causal, group != 4, one row block) plan as SHARED.
     const bool pair_forced = c->prefill_kernel == GQA_PREFILL_KERNEL_PAIRED && pairable;
     const int target = (pair_auto || pair_forced) ? 1 : c->prefill_wgs_opt > 0 ? c->prefill_wgs_opt
                        : segs > 0                 ? segs * shared_wgs
                                                   : c->n_cu;
-    PrefillPlan plan = plan_prefill(q_len, kv_span, c->group, c->cfg.n_kv_heads, target, kMaxPrefillSegs);
+    PrefillPlan plan = plan_for(target, kMaxPrefillSegs);
     float* const ws = plan_auto ? c->auto_ws : c->pre_ws;
-    const bool fits = prefill_workspace_floats(plan, q_len, c->cfg.n_q_heads, c->cfg.head_dim) <=
-                      (plan_auto ? c->auto_ws_floats : c->pre_ws_floats);
-    if (!fits) plan = plan_prefill(q_len, kv_span, c->group, c->cfg.n_kv_heads, 1, 1);  // one segment
-    const bool rows = c->prefill_kernel == GQA_PREFILL_KERNEL_ROWS || (plan_auto && (segs == 0 || !fits));
+    if (!plan_auto && prefill_workspace_floats(plan, q_len, c->cfg.n_q_heads, c->cfg.head_dim) > c->pre_ws_floats)
+        plan = plan_for(1, 1);  // one segment
+    const bool rows = c->prefill_kernel == GQA_PREFILL_KERNEL_ROWS || (plan_auto && segs == 0);
     PrefillArgs a{};
     const size_t seq_off = c->paged ? 0 : (size_t)b * c->cfg.n_kv_heads * c->l_cap * c->cfg.head_dim;
     a.q = (const uint16_t*)q;
@@ -616,7 +644,10 @@ int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_p
                       (c->prefill_kernel == GQA_PREFILL_KERNEL_AUTO && paired_wgs == c->n_cu))
                  ? 1 : 0;
     HIP_TRY(launch_prefill(c->cfg.head_dim, c->group, a, timed(c, GQA_TIMER_PREFILL, s)));
-    if (plan.n_segs > 1) HIP_TRY(launch_prefill_combine(c->cfg.head_dim, a, timed(c, GQA_TIMER_COMBINE, s)));
+    if (plan.n_segs > 1) {
+        HIP_TRY(launch_prefill_combine(c->cfg.head_dim, a, timed(c, GQA_TIMER_COMBINE, s)));
+        if (plan_auto && s != c->stream) HIP_TRY(hipEventRecord(c->ev_auto_ws, s));
+    }
     c->last_prefill_kernel = a.pair ? GQA_PREFILL_KERNEL_PAIRED : GQA_PREFILL_KERNEL_SHARED;
     c->last_prefill_segs = plan.n_segs;
     return GQA_OK;
@@ -1052,6 +1083,7 @@ int create_ctx(const gqa_config* cfg, int32_t page_size, int32_t n_pages, int32_
     if (rc == GQA_OK) {
         bool ok = hipEventCreate(&c->ev_begin) == hipSuccess && hipEventCreate(&c->ev_end) == hipSuccess;
         for (int i = 0; i < 4 && ok; ++i) ok = hipEventCreate(&c->ev_t[i]) == hipSuccess;
+        ok = ok && hipEventCreateWithFlags(&c->ev_auto_ws, hipEventDisableTiming | hipEventDisableSystemFence) == hipSuccess;
         for (hipEvent_t& e : c->ev_part) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
         if (!ok) rc = GQA_ERR_HIP;
     }
@@ -1244,6 +1276,7 @@ int gqa_destroy(gqa_ctx* c) {
     if (c->kv_pinned) (void)hipHostFree(c->kv_pinned);
     for (hipEvent_t e : c->ev_part)
         if (e) (void)hipEventDestroy(e);
+    if (c->ev_auto_ws) (void)hipEventDestroy(c->ev_auto_ws);
     if (c->ev_begin) (void)hipEventDestroy(c->ev_begin);
     if (c->ev_end) (void)hipEventDestroy(c->ev_end);
     for (int i = 0; i < GQA_TIMER_COUNT; ++i) {

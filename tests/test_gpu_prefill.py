@@ -653,3 +653,48 @@ def test_forced_segments_beside_automatic_ones(forced):
             torch.cuda.synchronize()
             for o, ref in zip(o_dev, refs):
                 check_rows(o.cpu().numpy().view(np.uint16), None, ref, None)
+
+
+def test_segment_workspace_follows_the_stream_in_use():
+    """Segments move to the stream that asks for them twice in a row: from the context's own (a host call) to a
+    caller's and on to another, each taken over with the owner's launches still in flight, and every output holds."""
+    torch = pytest.importorskip("torch")
+    import ctypes
+
+    from lara_amd import _lib
+
+    rng = np.random.default_rng(5400)
+    hq, hkv, d, q_len, kv_len, deep = 32, 8, 128, 16, 9000, 12
+    k, v = bf16_normal(rng, (hkv, kv_len, d)), bf16_normal(rng, (hkv, kv_len, d))
+    qs = [bf16_normal(rng, (hq, q_len, d)) for _ in range(2)]
+    refs = [oracle_for(q, k, v, causal=True, q_pos_base=kv_len - q_len)[0] for q in qs]
+    with AttentionAccelerator(max_seq_len=kv_len, max_q_len=64) as acc:
+        acc.load_kv(k, v)
+        q_dev = [torch.from_numpy(q.view(np.int16)).cuda() for q in qs]
+        o_dev = [[torch.zeros_like(q_dev[0]) for _ in range(deep)] for _ in range(2)]
+        torch.cuda.synchronize()
+
+        def launch(i, n, stream):
+            _lib.check(acc._lib.gqa_prefill_device(acc._ctx, 0, ctypes.c_void_p(q_dev[i].data_ptr()), q_len,
+                                                   kv_len - q_len, kv_len, 0, 1, ctypes.c_void_p(o_dev[i][n].data_ptr()),
+                                                   None, ctypes.c_void_p(stream) if stream else None), "prefill")
+            return acc.last_prefill_plan()
+
+        out = acc.prefill_chunk(qs[0], q_pos_base=kv_len - q_len, kv_len=kv_len)
+        assert acc.last_prefill_plan()[1] > 1
+        check_rows(out, None, refs[0], None)
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        handles = [None] + [s.cuda_stream for s in streams] + [None]
+        for old, new in zip(handles, handles[1:]):
+            print(f"[segments] from {old} to {new}", flush=True)
+            for o in o_dev[0] + o_dev[1]:
+                o.zero_()
+            torch.cuda.synchronize()
+            for n in range(deep):
+                assert launch(0, n, old)[1] > 1
+            plans = [launch(1, n, new) for n in range(deep)]
+            assert plans[0] == ("rows", 1) and all(segs > 1 for _, segs in plans[1:])
+            torch.cuda.synchronize()
+            for i in range(2):
+                for o in o_dev[i]:
+                    check_rows(o.cpu().numpy().view(np.uint16), None, refs[i], None)
