@@ -698,3 +698,17 @@ def test_segment_workspace_follows_the_stream_in_use():
             for i in range(2):
                 for o in o_dev[i]:
                     check_rows(o.cpu().numpy().view(np.uint16), None, refs[i], None)
+
+
+def test_loads_of_growing_length():
+    """gqa_load_kv from one row to more than its staging holds (8 MiB), each load longer than the last, into a cache
+    of exactly the rows of the longest and at an offset in a wider one."""
+    rng = np.random.default_rng(5500)
+    for cap, first in ((2304, 0), (4096, 65)):
+        with AttentionAccelerator(max_seq_len=cap, max_q_len=64) as acc:
+            for n in (1, 15, 16, 17, 240, 511, 512, 513, 2047, 2048, 2049, 2304):
+                print(f"[load] cap={cap} n={n}", flush=True)
+                k, v = bf16_normal(rng, (8, n, 128)), bf16_normal(rng, (8, n, 128))
+                acc.load_kv(k, v, start_pos=first)
+                kr, vr = acc.read_kv(0, first, n)
+                assert np.array_equal(kr, k) and np.array_equal(vr, v)
