@@ -40,6 +40,8 @@
 
 #include <math.h>
 
+#include <algorithm>
+
 #pragma clang fp contract(off)
 
 namespace lara {
@@ -263,10 +265,12 @@ __global__ __launch_bounds__(kRtlThreads, 2) void rtl_transaction_kernel(RtlArgs
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, half = lane >> 5;
-    const int hq = blockIdx.x;
+    const int n_t = (a.q_len + kTileRows - 1) / kTileRows;
+    const int lin = (int)(blockIdx.y * gridDim.x + blockIdx.x);  // heads fastest
+    if (lin >= n_t * a.n_q_heads) return;
+    const int hq = lin % a.n_q_heads, by = lin / a.n_q_heads;
     // Row tile: longest first, or, in a grid that is resident at once (two work-groups per CU), the
     // shortest beside the longest (512 rows x 32 heads, causal: 76.6 us against 81.9).
-    const int n_t = gridDim.y, by = blockIdx.y;
     const int t = a.pair_tiles && by >= (n_t + 1) / 2 ? by - (n_t + 1) / 2 : n_t - 1 - by;
     const int hk = hq / (a.n_q_heads / a.n_kv_heads);
     const uint16_t* kb = a.kc + (size_t)hk * a.l_cap * D;
@@ -566,8 +570,13 @@ __global__ __launch_bounds__(kRtlThreads, 2) void rtl_transaction_kernel(RtlArgs
 
 hipError_t launch_rtl_transaction(int head_dim, const RtlArgs& args, int n_cu, const Launch& l) {
     RtlArgs a = args;
-    const dim3 grid(a.n_q_heads, (a.q_len + kTileRows - 1) / kTileRows), block(kRtlThreads);
-    a.pair_tiles = (int64_t)grid.x * grid.y <= 2 * (int64_t)n_cu;
+    // The (tile, head) pairs in rows of at most 2^16 work-groups (an axis of the grid holds 2^32 threads, y and z 65535
+    // work-groups).
+    const int64_t pairs = (int64_t)a.n_q_heads * ((a.q_len + kTileRows - 1) / kTileRows);
+    const int64_t per_row = std::min<int64_t>(pairs, 1 << 16), rows = (pairs + per_row - 1) / per_row;
+    if (pairs + per_row > INT32_MAX) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)per_row, (unsigned)rows), block(kRtlThreads);
+    a.pair_tiles = pairs <= 2 * (int64_t)n_cu;
     if (head_dim == 128) return launch_kernel(rtl_transaction_kernel<128>, grid, block, l, a);
     if (head_dim == 64) return launch_kernel(rtl_transaction_kernel<64>, grid, block, l, a);
     return hipErrorInvalidValue;

@@ -6,6 +6,7 @@ independent implementations of the same bit-level contract; every output word mu
 import numpy as np
 import pytest
 
+from lara_amd import _lib
 from lara_amd.attn_driver import AttentionAccelerator
 from oracle import gqa_oracle as orc
 from oracle import rtl_exact as rtl
@@ -218,3 +219,22 @@ def test_kv260_mode_infinite_o_word_forgotten(d):
             assert np.any(want[:, 18 * 16:19 * 16] & 0x7F80 == 0x7F80) == causal and not np.any(want[:, -1] & 0x7F80 == 0x7F80)
             mism = np.argwhere(out != want)
             assert mism.size == 0, f"{len(mism)} mismatching words, first at {tuple(mism[0])}"
+
+
+@pytest.mark.parametrize("L", [65535 * 32, 65535 * 32 + 1, 65536 * 32 + 33])
+def test_kv260_mode_more_row_tiles_than_a_grid_axis_holds(L):
+    """Prompts of 65535 32-row tiles and more, up to a second row of the grid: 64 rows repeated, every repetition
+    equal to the oracle's words of the first."""
+    print(f"[kv260] L={L}", flush=True)
+    rng = np.random.default_rng(2800)
+    q, k, v = (bf16_normal(rng, (1, 64, 64)) for _ in range(3))
+    want, _, _ = rtl.attention(q, k, v, causal=False)
+    tiled = np.ascontiguousarray(np.resize(q[0], (L, 64))[None])
+    with AttentionAccelerator(n_q_heads=1, n_kv_heads=1, head_dim=64, max_seq_len=64, max_q_len=L, numerics="kv260") as acc:
+        acc.load_kv(k, v)
+        out = np.empty_like(tiled)  # (the driver's own positions end at the board's 16 bits)
+        acc._call("gqa_prefill", 0, _lib.as_u16_ptr(tiled), L, 0, 64, 0, 0, _lib.as_u16_ptr(out), None)
+    assert np.array_equal(out[0, :64], want[0])
+    whole = L // 64 * 64
+    assert np.array_equal(out[0, :whole].reshape(-1, 64, 64), np.broadcast_to(out[0, :64], (whole // 64, 64, 64)))
+    assert np.array_equal(out[0, whole:], out[0, :L - whole])
