@@ -510,9 +510,7 @@ class AttentionAccelerator:
         ``TimeoutError`` when ``timeout_ms`` expires.
         """
         self._ensure_open()
-        status = self.status()
-        if status & (STATUS_ERROR | STATUS_STREAM_ERROR):
-            raise RuntimeError(f"accelerator error status=0x{status:08x}, code=0x{self._error_code:02x}")
+        self._raise_on_error_status()
         rc = self._lib.gqa_wait(self._ctx, -1 if timeout_ms is None else int(timeout_ms))
         if rc == _lib.GQA_ERR_TIMEOUT:
             raise TimeoutError("attention accelerator timed out while servicing load requests")
@@ -761,19 +759,30 @@ class AttentionAccelerator:
                        _lib.as_u16_ptr(out), lse_ptr)
         return (out, lse) if return_lse else out
 
+    def _raise_on_error_status(self) -> None:
+        status = self.status()
+        if status & (STATUS_ERROR | STATUS_STREAM_ERROR):
+            raise RuntimeError(f"accelerator error status=0x{status:08x}, code=0x{self._error_code:02x}")
+
     def _finish_transaction(self, prof: RunProfile, L: int, timeout_ms: int | None):
         """Wait for the started transaction and copy its output: (words, perf counters).  Without a timeout the
-        read-back starts at once and takes the output as it arrives; the wait is then the time before the device's
-        own output copy (its share of the read-back is ``output_dma_transfer_ms`` either way)."""
+        read-back starts at once and takes the output as it arrives; an error then is the one ``wait_done`` reports."""
         t = time.perf_counter()
         if timeout_ms is not None:
             self.wait_done(None, None, None, L, timeout_ms=timeout_ms)
             prof.request_service_ms = (time.perf_counter() - t) * 1000.0
             t = time.perf_counter()
-        words = self.readback_o(L)
+            words = self.readback_o(L)
+        else:
+            self._raise_on_error_status()
+            try:
+                words = self.readback_o(L)
+            except _lib.GqaError as exc:
+                if exc.code == _lib.GQA_ERR_RESULT_LEN:
+                    raise
+                self._error_code = exc.code
+                raise RuntimeError(f"accelerator error status=0x{self.status():08x}, code=0x{exc.code:02x}") from exc
         elapsed_ms = (time.perf_counter() - t) * 1000.0
-        if timeout_ms is None:
-            self.wait_done(None, None, None, L)  # error status, if any, as wait_done reports it
         perf = self.read_perf()
         if timeout_ms is None:
             copy_ms = perf["stall_cycles"] / (self._pl_clock_mhz * 1000.0) if self._pl_clock_mhz > 0 else 0.0

@@ -1,7 +1,10 @@
 """Host-side logic of the drop-in driver and the roofline model (no GPU needed)."""
+import ctypes
+
 import numpy as np
 import pytest
 
+from lara_amd import _lib
 from lara_amd import attn_driver as drv
 from lara_amd import benchmark as bm
 from oracle import gqa_oracle as orc
@@ -122,3 +125,47 @@ def test_report_metrics_closed_forms():
     assert e["max_relative_floor_1e-6"] == 1.0
     env = bm.collect_environment()
     assert env["os_cpu_count"] >= 1 and "thread_environment" in env
+
+
+class _FakeDevice:
+    """The calls that finish a transaction, with a status each: an output copy of 3 of 9 ticks at 1 MHz."""
+
+    def __init__(self, read=_lib.GQA_OK, wait=_lib.GQA_OK):
+        self.read, self.wait = read, wait
+
+    def gqa_status(self, ctx, word):
+        return _lib.GQA_OK
+
+    def gqa_wait(self, ctx, timeout_ms):
+        return self.wait
+
+    def gqa_read_output(self, ctx, out, n_words):
+        return self.read
+
+    def gqa_read_perf(self, ctx, total, kernel, copy, mhz):
+        total._obj.value, kernel._obj.value, copy._obj.value, mhz._obj.value = 9, 5, 3, 1.0
+        return _lib.GQA_OK
+
+
+def _finished(device, timeout_ms):
+    acc = drv.AttentionAccelerator.__new__(drv.AttentionAccelerator)
+    acc._lib, acc._ctx, acc._closed, acc._error_code = device, ctypes.c_void_p(), False, drv.ERR_NONE
+    acc.n_q_heads, acc.head_dim = 2, 64
+    prof = drv.RunProfile("t", "g", None, 1.0, 16, True, 0, 0)
+    try:
+        acc._finish_transaction(prof, 16, timeout_ms)
+    except Exception as exc:
+        acc._closed = True
+        return acc, prof, exc
+    acc._closed = True
+    return acc, prof, None
+
+
+@pytest.mark.parametrize("timeout_ms", [None, 100])
+def test_transaction_error_is_the_one_wait_done_reports(timeout_ms):
+    for code in (_lib.GQA_ERR_HIP, _lib.GQA_ERR_NO_TRANSACTION):
+        device = _FakeDevice(read=code) if timeout_ms is None else _FakeDevice(wait=code)
+        acc, _, exc = _finished(device, timeout_ms)
+        assert type(exc) is RuntimeError and f"code=0x{code:02x}" in str(exc) and acc._error_code == code
+    acc, _, exc = _finished(_FakeDevice(read=_lib.GQA_ERR_RESULT_LEN), timeout_ms)
+    assert isinstance(exc, _lib.GqaError) and acc._error_code == drv.ERR_RESULT_LEN
