@@ -233,7 +233,9 @@ class RunProfile:
     """Per-transaction timing record; field names follow sw/attn_driver.py:207-247.
 
     On the GPU the ``pl_*`` cycle fields count device-clock ticks at ``clock_mhz``:
-    total = copy-in to copy-out, mac = attention kernels, stall = output copy.
+    total = copy-in to copy-out, mac = attention kernels, stall = output copy.  The time from the start to the
+    output in the caller's array is ``output_dma_transfer_ms``, the device's output copy, and
+    ``request_service_ms``, the rest.
     """
 
     timestamp_utc: str
@@ -770,8 +772,6 @@ class AttentionAccelerator:
         t = time.perf_counter()
         if timeout_ms is not None:
             self.wait_done(None, None, None, L, timeout_ms=timeout_ms)
-            prof.request_service_ms = (time.perf_counter() - t) * 1000.0
-            t = time.perf_counter()
             words = self.readback_o(L)
         else:
             self._raise_on_error_status()
@@ -784,11 +784,9 @@ class AttentionAccelerator:
                 raise RuntimeError(f"accelerator error status=0x{self.status():08x}, code=0x{exc.code:02x}") from exc
         elapsed_ms = (time.perf_counter() - t) * 1000.0
         perf = self.read_perf()
-        if timeout_ms is None:
-            copy_ms = perf["stall_cycles"] / (self._pl_clock_mhz * 1000.0) if self._pl_clock_mhz > 0 else 0.0
-            prof.request_service_ms = max(elapsed_ms - copy_ms, 0.0)
-            elapsed_ms -= prof.request_service_ms
-        prof.output_dma_transfer_ms = elapsed_ms
+        copy_ms = perf["stall_cycles"] / (self._pl_clock_mhz * 1000.0) if self._pl_clock_mhz > 0 else 0.0
+        prof.output_dma_transfer_ms = min(copy_ms, elapsed_ms)
+        prof.request_service_ms = elapsed_ms - prof.output_dma_transfer_ms
         return words, perf
 
     def run_attention(

@@ -169,3 +169,12 @@ def test_transaction_error_is_the_one_wait_done_reports(timeout_ms):
         assert type(exc) is RuntimeError and f"code=0x{code:02x}" in str(exc) and acc._error_code == code
     acc, _, exc = _finished(_FakeDevice(read=_lib.GQA_ERR_RESULT_LEN), timeout_ms)
     assert isinstance(exc, _lib.GqaError) and acc._error_code == drv.ERR_RESULT_LEN
+
+
+@pytest.mark.parametrize("timeout_ms", [None, 100])
+def test_transaction_profile_splits_the_wait_at_the_device_copy(timeout_ms, monkeypatch):
+    clock = iter((10.0, 10.5))  # 500 ms from the start to the words; the device's copy: 3 ticks at 1 MHz
+    monkeypatch.setattr(drv.time, "perf_counter", lambda: next(clock))
+    _, prof, exc = _finished(_FakeDevice(), timeout_ms)
+    assert exc is None
+    assert prof.output_dma_transfer_ms == pytest.approx(0.003) and prof.request_service_ms == pytest.approx(499.997)
