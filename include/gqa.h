@@ -422,6 +422,10 @@ int gqa_synchronize(gqa_ctx* ctx);
  * chosen per launch, and tests use this to check which decomposition a launch took. */
 int gqa_last_prefill_plan(gqa_ctx* ctx, int32_t* kernel, int32_t* n_segs);
 
+/* gqa_last_prefill_row_heads: the query heads per work-group of that launch (1 or 2) where it was
+ * GQA_PREFILL_KERNEL_ROWS, else 0. */
+int gqa_last_prefill_row_heads(gqa_ctx* ctx, int32_t* heads);
+
 #ifdef __cplusplus
 }
 #endif

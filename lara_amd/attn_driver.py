@@ -596,6 +596,12 @@ class AttentionAccelerator:
                  _lib.GQA_PREFILL_KERNEL_PAIRED: "paired"}
         return names.get(int(kernel.value), ""), int(segs.value)
 
+    def last_prefill_row_heads(self) -> int:
+        """Query heads per work-group of the last prefill launch in row blocks (1 or 2; 0 after any other)."""
+        heads = ctypes.c_int32(0)
+        self._call("gqa_last_prefill_row_heads", ctypes.byref(heads))
+        return int(heads.value)
+
     def page_info(self) -> dict[str, int]:
         """Page size, pool size, free pages and block-table width of a paged engine."""
         vals = [ctypes.c_int32(0) for _ in range(4)]

@@ -137,6 +137,7 @@ struct gqa_ctx {
     PageTable pages;
     int last_prefill_kernel = 0;  // decomposition and KV segments of the last prefill launch (gqa_last_prefill_plan)
     int last_prefill_segs = 0;
+    int last_prefill_row_heads = 0;  // query heads per work-group of a launch in row blocks
 };
 
 // A prepared decode step (gqa_graph_capture_decode_append): the launch description planned once,
@@ -634,6 +635,7 @@ int run_prefill(gqa_ctx* c, int32_t b, const void* q, int32_t q_len, int32_t q_p
         a.rows_heads = rows_two_heads(q_len, kv_span, causal != 0, c->group, c->cfg.n_kv_heads, c->cfg.head_dim, c->n_cu) ? 2 : 1;
         HIP_TRY(launch_prefill_rows(c->cfg.head_dim, a, timed(c, GQA_TIMER_PREFILL, s)));
         c->last_prefill_kernel = GQA_PREFILL_KERNEL_ROWS;
+        c->last_prefill_row_heads = a.rows_heads;
         c->last_prefill_segs = 1;
         return GQA_OK;
     }
@@ -2133,6 +2135,12 @@ int gqa_last_prefill_plan(gqa_ctx* c, int32_t* kernel, int32_t* n_segs) {
     if (!c || !kernel || !n_segs) return GQA_ERR_NULL;
     *kernel = c->last_prefill_kernel;
     *n_segs = c->last_prefill_segs;
+    return GQA_OK;
+}
+
+int gqa_last_prefill_row_heads(gqa_ctx* c, int32_t* heads) {
+    if (!c || !heads) return GQA_ERR_NULL;
+    *heads = c->last_prefill_kernel == GQA_PREFILL_KERNEL_ROWS ? c->last_prefill_row_heads : 0;
     return GQA_OK;
 }
 

@@ -12,9 +12,12 @@ Bars (the stage specification is in oracle/layer_oracle.py):
   chain (rounding to bf16 at the same points); with KV260 numerics, word for word equal to
   the C restatement of the board arithmetic on the GPU's Q/K/V.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
+from lara_amd import _lib
 from lara_amd.attn_driver import AttentionAccelerator
 from oracle import gqa_oracle as orc
 from oracle import layer_oracle as lo
@@ -315,3 +318,53 @@ def test_few_tokens_stage_keeps_the_general_calls():
             torch.cuda.synchronize()
             got = host(dst).reshape(8, L, 128)
             assert_same_stage(got, want[0])
+
+
+def _stage_launches(acc):
+    """Launches of the stages since profiling was switched on: (RMSNorm, projection, RoPE)."""
+    counts = (ctypes.c_int32 * _lib.GQA_TIMER_COUNT)()
+    _lib.check(acc._lib.gqa_kernel_launch_counts(acc._ctx, counts, _lib.GQA_TIMER_COUNT), "counts")
+    return tuple(int(counts[t]) for t in (_lib.GQA_TIMER_NORM, _lib.GQA_TIMER_PROJECTION, _lib.GQA_TIMER_ROPE))
+
+
+@pytest.mark.parametrize("hidden,L,hq,hkv,d,one", [(1024, 16, 8, 2, 64, True), (2048, 3, 16, 8, 128, True),
+                                                   (4096, 16, 32, 8, 128, True), (4096, 17, 32, 8, 128, False),
+                                                   (8192, 8, 64, 8, 128, True), (8192, 9, 8, 2, 128, False),
+                                                   (3072, 4, 8, 2, 128, False)])
+def test_few_tokens_stage_is_one_launch(hidden, L, hq, hkv, d, one):
+    """Up to 16 tokens (8 at hidden 8192) of a hidden size that has one take one launch, timed as the projection;
+    the others RMSNorm, the library's product and RoPE."""
+    print(f"[layer] launches hidden={hidden} L={L} hq={hq} hkv={hkv}", flush=True)
+    rng = np.random.default_rng(hidden + L)
+    wq, wk, wv = weights(rng, hq * d, hkv * d, hidden)
+    gamma = orc.fp32_to_bf16_u16(np.ones(hidden, np.float32))
+    with AttentionAccelerator(n_q_heads=hq, n_kv_heads=hkv, head_dim=d, max_seq_len=64) as acc:
+        _lib.check(acc._lib.gqa_set_option(acc._ctx, _lib.GQA_OPT_PROFILE, 1), "profile")
+        stage(acc, bf16_normal(rng, (L, hidden)), wq, wk, wv, gamma)
+        assert _stage_launches(acc) == ((0, 1, 0) if one else (1, 1, 1))
+
+
+@pytest.mark.parametrize("hidden,L,hq,hkv", [(4096, 2, 64, 8), (1024, 3, 128, 16), (2048, 1, 100, 50),
+                                             (1024, 16, 128, 64), (8192, 2, 128, 16)])
+def test_few_tokens_stage_of_many_tiles(hidden, L, hq, hkv):
+    """Work-groups of 2 to 8 output tiles in turn (on 256 CUs: 640, 1280, 1600 and 2048 tiles of 16 rows; 8192: two
+    chunks of the product each), odd counts of chunks among them: every projected row within its fp32 bound, RoPE
+    word for word, in one launch."""
+    d = 128
+    print(f"[layer] many tiles hidden={hidden} L={L} hq={hq} hkv={hkv}", flush=True)
+    rng = np.random.default_rng(hidden + hq + L)
+    x = bf16_normal(rng, (L, hidden))
+    wq, wk, wv = weights(rng, hq * d, hkv * d, hidden)
+    with AttentionAccelerator(n_q_heads=hq, n_kv_heads=hkv, head_dim=d, max_seq_len=64) as acc:
+        _lib.check(acc._lib.gqa_set_option(acc._ctx, _lib.GQA_OPT_PROFILE, 1), "profile")
+        plain = stage(acc, x, wq, wk, wv, None, rope=False, row0=3)
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            assert _stage_launches(acc) == (0, 1, 0)
+        roped = stage(acc, x, wq, wk, wv, None, row0=3, q_pos_base=901, kv_pos_base=3)
+    for g, w, H in zip(plain, (wq, wk, wv), (hq, hkv, hkv)):
+        got = orc.bf16_u16_to_fp32(g).astype(np.float64).transpose(1, 0, 2).reshape(L, H * d)
+        err = np.abs(got - lo.project_exact(x, w))
+        bound = lo.projection_error_bound(x, w)
+        assert np.all(err <= bound), float(np.max(err / bound))
+    assert np.array_equal(roped[0], lo.apply_rope(plain[0], 901))
+    assert np.array_equal(roped[1], lo.apply_rope(plain[1], 3)) and np.array_equal(roped[2], plain[2])

@@ -370,9 +370,8 @@ def test_prefill_segmentation_invariance(wgs):
 
 @pytest.mark.parametrize("v_scale", [1e30, 1e-30, 1e-39, "mixed", "weighted"])
 def test_segment_partials_at_extreme_magnitudes(v_scale):
-    """KV segments hand their rows to the merge as fp16 O / l divided by the row's largest
-    |O / l|: outputs of very large or very small magnitude, and rows mixing both, keep the
-    2-ulp bound with many segments."""
+    """KV segments hand their un-normalised rows to the merge in fp32: outputs of very large or
+    very small magnitude, and rows mixing both, keep the 2-ulp bound with many segments."""
     seeds = {"mixed": 500, "weighted": 501}
     rng = np.random.default_rng(seeds.get(v_scale) or int(np.log10(v_scale)) + 600)
     q_len, kv_len = 128, 1024
@@ -558,10 +557,12 @@ def test_row_blocks_of_two_heads(hq, hkv, q_len, history, causal, paged):
         print(f"[two heads] {hq}/{hkv} {q_len} after {history}", flush=True)
         out, lse = acc.prefill_chunk(q, q_pos_base=history, kv_len=L, k_rows=k[:, history:], v_rows=v[:, history:],
                                      causal=causal, return_lse=True)
+        assert acc.last_prefill_row_heads() == 2
         kr, vr = acc.read_kv(0, 0, L)
         assert np.array_equal(kr, k) and np.array_equal(vr, v)
         for at in range(0, q_len, 64):
             o1, l1 = acc.prefill_chunk(q[:, at:at + 64], q_pos_base=history + at, kv_len=L, causal=causal, return_lse=True)
+            assert acc.last_prefill_row_heads() == 1
             assert np.array_equal(out[:, at:at + 64], o1)
             assert np.array_equal(lse[:, at:at + 64].view(np.uint32), l1.view(np.uint32))
     ref, ref_lse = oracle_for(q, k, v, causal=causal, q_pos_base=history)
