@@ -65,9 +65,9 @@ extern "C" {
 /* Tunables for gqa_set_option. */
 #define GQA_OPT_DECODE_CHUNK 1 /* keys per split-KV work-group (a multiple of 64 giving at most max(l_cap / 256,
                                   the automatic plan's) splits; a last split of <= chunk/4 keys joins the one
-                                  before it; 0 = auto: about 8 waves per CU, whole 16-key rounds per wave, or
-                                  in 64-key steps about 112 work-groups per 256 CUs where K/V of at most
-                                  16 MiB would need a merge launch and merge in the decode launch that way).
+                                  before it; 0 = auto: about 8 waves per CU, whole 16-key rounds per wave, or,
+                                  for K/V of at most 16 MiB, in 64-key steps about 112 work-groups per 256 CUs
+                                  that merge in the decode launch).
                                   The automatic plan does not split a (sequence, kv head) whose K/V take
                                   at most 128 KiB (256 KiB from 32 of them on).  Work-groups have 8 waves, or
                                   4 when the 8-wave plan has at most 8 work-groups (the automatic chunk is

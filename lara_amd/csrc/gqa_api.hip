@@ -271,12 +271,14 @@ constexpr int64_t kSmallDecodeGrid = 8;
 // 8/2 heads of 64, 576 keys 9.1 against 8.3 by a launch; one of 6000, 32/8 heads, 448 keys 8.2 against 8.1).
 // Groups above 8 take longer per key and merge: up to kFusedPlanKeysWide keys they still save other streams more
 // (7 of 200 .. 3000, 32/2 heads of 64, 7.1 / 10.3 against 5.9 / 11.1), beyond not (8 of 4096 7.5 / 9.9 against 7.9 / 11.5).
-// (The byte bound ends it before the keys do at D 128 alone.)  A plan that
-// merges in-launch as it is stays: its shorter splits are the better ones for sequences that end well before the
-// capacity (one of 1000 keys in 4096 rows, 64/8 heads of 128: 9.7 in splits of 256, 10.1 of 320; one of 300 there,
-// 32/2 heads of 64: 5.7 in splits of 256, 8.0 of 128).  So does a grid that needs a merge launch at any size: 208
-// work-groups instead of 256 to 264 gained at full caches (3 of 8000, 64/8 heads, 25.7 -> 21.0 on one stream) but lost as
-// much at a quarter of the capacity (3 of 2500 in 10000 rows 16.2 -> 20.7).
+// (The byte bound ends it before the keys do at D 128 alone.)
+// A plan that merges in-launch as it is takes longer splits this way at D 128 only, for the CUs that it leaves to other
+// launches (a layer's step of one token over 2048 keys, 32/8 heads, 18.5 -> 16.5 over three streams; one of 4096 keys
+// 7.3 / 8.9 -> 6.6 / 8.8), at up to 0.5 us where the sequence ends well before the capacity (one of 1000 keys in 4096
+// rows 7.6 -> 8.1 on one stream); never shorter ones (one of 300 keys in 4096 rows, 32/2 heads of 64: 5.7 in splits of
+// 256, 8.0 of 128).  Grids that need a merge launch at any size stay, too: 208 work-groups instead of 256 to 264
+// gained at full caches (3 of 8000, 64/8 heads, 25.7 -> 21.0 on one stream) but lost as much at a quarter of the
+// capacity (3 of 2500 in 10000 rows 16.2 -> 20.7).
 constexpr int64_t kFusedPlanBytes = 16 << 20;
 constexpr int kFusedPlanUnits = 32, kFusedPlanSplits = 32;
 constexpr int kFusedPlanKeys = 448, kFusedPlanKeysWide = 384;  // (wide: groups above 8)
@@ -302,19 +304,23 @@ DecodeShape plan_decode_shape(int batch, int n_kv_heads, int group, int head_dim
     };
     const DecodeShape big = shape(kDecodeWaves);
     if (units * big.max_splits <= kSmallDecodeGrid) return shape(kDecodeWavesSmall);
-    if (chunk_opt > 0 || merge_option != GQA_DECODE_MERGE_AUTO || big.max_splits <= 1 || big.fused) return big;
+    if (chunk_opt > 0 || merge_option != GQA_DECODE_MERGE_AUTO || big.max_splits <= 1) return big;
     const int shortest = kDecodeWaves * decode_round_keys(group);
-    if (big.chunk == shortest) {
+    DecodeShape plain = big;
+    if (!big.fused && big.chunk == shortest) {
         const DecodeShape twice = in_chunks(2 * shortest, kDecodeWaves);
-        if (twice.fused) return twice;
+        if (twice.fused) plain = twice;
     }
-    if (units > kFusedPlanUnits || units * max_len * head_dim * 2 * 2 > kFusedPlanBytes) return big;
+    if (units > kFusedPlanUnits || units * max_len * head_dim * 2 * 2 > kFusedPlanBytes || (plain.fused && head_dim <= 64))
+        return plain;
     const int splits = std::max(1, std::min(kFusedPlanSplits, (int)(kFusedPlanGrid * n_cu) / (int)units));
     const int even = (max_len + splits - 1) / splits;
     DecodeShape s = in_chunks(std::max(shortest, (even + kChunkOptionQuantum - 1) / kChunkOptionQuantum * kChunkOptionQuantum),
                               kDecodeWaves);
     s.fused = s.max_splits > 1 && s.max_splits <= kFusedPlanSplits && 2 * units * s.max_splits <= n_cu;
-    return s.fused && s.chunk <= (group > 8 ? kFusedPlanKeysWide : kFusedPlanKeys) ? s : big;
+    const bool take = s.fused && s.chunk <= (group > 8 ? kFusedPlanKeysWide : kFusedPlanKeys) &&
+                      !(plain.fused && s.chunk <= plain.chunk);
+    return take ? s : plain;
 }
 
 constexpr int kProfileLaunches = 512;  // event pairs kept per timer slot
