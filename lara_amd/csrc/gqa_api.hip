@@ -1007,6 +1007,28 @@ size_t prefill_workspace_need(const gqa_ctx* c, int target_wgs) {
     return need;
 }
 
+// The forced launches' workspace for a work-group target (kept if it already suffices).
+int grow_forced_workspace(gqa_ctx* c, int target_wgs) {
+    const size_t need = prefill_workspace_need(c, target_wgs);
+    if (need <= c->pre_ws_floats) return GQA_OK;
+    if (c->pre_ws) {  // launches may be using it
+        const int rc = txn_idle(c);
+        if (rc != GQA_OK) return rc;
+        HIP_TRY(hipSetDevice(c->cfg.device));
+        HIP_TRY(hipDeviceSynchronize());
+    }
+    HIP_TRY(hipSetDevice(c->cfg.device));
+    float* ws = nullptr;
+    if (hipMalloc(&ws, need * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();
+        return GQA_ERR_OOM;
+    }
+    (void)hipFree(c->pre_ws);
+    c->pre_ws = ws;
+    c->pre_ws_floats = need;
+    return GQA_OK;
+}
+
 int create_ctx(const gqa_config* cfg, int32_t page_size, int32_t n_pages, int32_t n_layers, gqa_ctx** out_ctx) {
     if (!cfg || !out_ctx) return GQA_ERR_NULL;
     *out_ctx = nullptr;
@@ -1069,9 +1091,7 @@ int create_ctx(const gqa_config* cfg, int32_t page_size, int32_t n_pages, int32_
     alloc((void**)&c->part_ml, units * c->max_splits_cap * group * 2 * sizeof(float));
     alloc((void**)&c->arrivals, (units + 1) * sizeof(int32_t));
     if (prefill_supported(k.head_dim, group)) {
-        c->pre_ws_floats = prefill_workspace_need(c, c->n_cu);
-        if (c->pre_ws_floats > 0) alloc((void**)&c->pre_ws, c->pre_ws_floats * sizeof(float));
-        if (k.max_seq_len > kAutoSegmentKeys) c->auto_ws_floats = c->pre_ws_floats;
+        if (k.max_seq_len > kAutoSegmentKeys) c->auto_ws_floats = prefill_workspace_need(c, c->n_cu);
         if (c->auto_ws_floats > 0) alloc((void**)&c->auto_ws, c->auto_ws_floats * sizeof(float));
     }
     alloc((void**)&c->q_dev, c->stage_words * 2);
@@ -1346,6 +1366,10 @@ int gqa_set_option(gqa_ctx* c, int32_t option, int64_t value) {
             if (value != GQA_PREFILL_KERNEL_AUTO && value != GQA_PREFILL_KERNEL_SHARED &&
                 value != GQA_PREFILL_KERNEL_ROWS && value != GQA_PREFILL_KERNEL_PAIRED)
                 return GQA_ERR_RANGE;
+            // (Where its workspace cannot be had, a forced kernel's launches take one segment.)
+            if ((value == GQA_PREFILL_KERNEL_SHARED || value == GQA_PREFILL_KERNEL_PAIRED) &&
+                prefill_supported(c->cfg.head_dim, c->group))
+                (void)grow_forced_workspace(c, c->prefill_wgs_opt > 0 ? c->prefill_wgs_opt : c->n_cu);
             c->prefill_kernel = (int)value;
             return GQA_OK;
         case GQA_OPT_DECODE_MERGE:
@@ -1373,19 +1397,9 @@ int gqa_set_option(gqa_ctx* c, int32_t option, int64_t value) {
                 c->prefill_wgs_opt = (int)value;
                 return GQA_OK;
             }
-            // Grow the segment workspace for the new target (kept if it already suffices).
-            const size_t need = prefill_workspace_need(c, value > 0 ? (int)value : c->n_cu);
-            if (need > c->pre_ws_floats) {
-                int rc = txn_idle(c);
-                if (rc != GQA_OK) return rc;
-                HIP_TRY(hipSetDevice(c->cfg.device));
-                HIP_TRY(hipDeviceSynchronize());
-                float* ws = nullptr;
-                if (hipMalloc(&ws, need * sizeof(float)) != hipSuccess) return GQA_ERR_OOM;
-                (void)hipFree(c->pre_ws);
-                c->pre_ws = ws;
-                c->pre_ws_floats = need;
-            }
+            const bool forced = c->prefill_kernel == GQA_PREFILL_KERNEL_SHARED || c->prefill_kernel == GQA_PREFILL_KERNEL_PAIRED;
+            const int rc = value > 0 || forced ? grow_forced_workspace(c, value > 0 ? (int)value : c->n_cu) : GQA_OK;
+            if (rc != GQA_OK) return rc;
             c->prefill_wgs_opt = (int)value;
             return GQA_OK;
         }
