@@ -256,10 +256,12 @@ __device__ __forceinline__ float wave_sum(float x) {
 // tokens, from LDS).  Two chunks of R loads each (256 KiB per CU) are in flight from the first
 // instructions on, across tiles, behind the loads of x only, which the norm waits for; the norm and
 // the rotations are done while the first weights arrive.  The waves' partial products meet in LDS.
-// Back to back over three sets of weights, hidden 4096, 32/8 heads of 128 (a streaming read of the weights alone:
-// 8.3 us): one token 10.7 us, 4: 11.1, 16: 14.3; norm, library product and RoPE launch took 17.5.  Hidden
-// 2048, 16/8 heads: 5.2 .. 8.2 against 17.3.  Hidden 8192, 64/8 heads (24.9 us): 28.6 .. 31.9 against
-// 30.5 .. 32.6.  (Two resident 16-row work-groups per CU with their own norms instead: 14.0, 5.3 and 48.3.)
+// us a launch on one stream / over three, back to back over 1 GiB of weight sets (more than any cache holds), norm,
+// library product and RoPE against this: hidden 4096, 32/8 heads of 128 (a streaming read of the weights alone 8.7):
+// one token 19.0 / 16.6 against 15.3 / 12.7, 4: 19.7 / 16.4 against 15.8 / 11.6, 16: 21.7 / 16.2 against 19.2 / 14.7;
+// hidden 2048, 16/8 heads (4.2): 16.6 / 16.1 against 7.3 / 5.7 (one) .. 10.2 / 8.6 (16); hidden 8192, 64/8 heads
+// (25.3): 41.8 / 31.1 against 37.9 / 28.9 (one) .. 43.2 / 32.9 against 41.2 / 32.1 (8).
+// (Two resident 16-row work-groups per CU with their own norms, one token over three streams: 14.0, 5.3 and 48.3.)
 template <int HIDDEN>
 struct FewTokensLds {
     static constexpr int kRow = HIDDEN / 8 + 4;  // 16-byte chunks of a row, shifted by 4 per token (bank conflicts)
@@ -479,7 +481,8 @@ bool few_tokens_supported(const FewTokensArgs& a, int n_cu) {
                             reinterpret_cast<uintptr_t>(a.w[0]) | reinterpret_cast<uintptr_t>(a.w[1]) |
                             reinterpret_cast<uintptr_t>(a.w[2]);
     return a.rope.n_tokens >= 1 && a.rope.n_tokens <= few_tokens_most(a.hidden) && a.rope.head_dim % kTileOut == 0 &&
-           (align & 15) == 0 && few_tokens_tiles(a) <= kFewWaves * n_cu && (a.hidden == 1024 || a.hidden == 2048 || a.hidden == 4096 || a.hidden == 8192);
+           (align & 15) == 0 && few_tokens_tiles(a) <= kFewWaves * n_cu &&
+           (a.hidden == 1024 || a.hidden == 2048 || a.hidden == 4096 || a.hidden == 8192);
 }
 
 hipError_t launch_few_tokens(const FewTokensArgs& a, int n_cu, const Launch& l) {

@@ -221,12 +221,11 @@ constexpr int kScoreRow = kSpanKeys + 4;       // LDS row of scores, padded agai
 
 // Words whose products and partial sums stay normal: zero, or a bf16 exponent in [71, 160].  Products
 // of two such words are multiples of 2^-126 (2 * (71 - 127 - 7)), so a partial sum is zero or normal, and
-// below 2^70, so no sum overflows.  The softmax weights (0, or 2^-12 .. 1) lie within.
+// below 2^75 (128 products below 2^68), so no sum overflows.  The softmax weights (0, or 2^-12 .. 1) lie within.
 constexpr uint32_t kRangeLo = 71u << 7, kRangeHi = (160u << 7) | 0x7Fu;
 
-// Normal values, and normal values or zero: native operations on them with such a result round as the
+// Normal values or zero: native operations on them with such a result round as the
 // board's (the sign of a zero apart).
-__device__ __forceinline__ bool normal_f(float x) { return __builtin_amdgcn_classf(x, 0x108); }
 __device__ __forceinline__ bool tame_f(float x) { return __builtin_amdgcn_classf(x, 0x168); }
 
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
