@@ -459,7 +459,8 @@ bool rows_two_heads(int q_len, int kv_span, bool causal, int group, int n_kv_hea
 // segments 7.5 at least, the host's two launches).
 // (Row blocks of two heads: the share of a round they fill times 8 + 2.15 per 256 keys.)
 // Segments have to save 4 of the first (the second launch costs the host more than a stream shows) and
-// must not lose the second.  So rows stay for short histories (32/8 heads, 100 rows after 4000 keys: 25.1 us
+// must not lose the second; one segment has to save 0.25, which keeps the row blocks for prompts of one key
+// block, where both estimates meet (8 rows, 8/2 heads of 64: 4.1 us of kernel against 4.6 shared).  So rows stay for short histories (32/8 heads, 100 rows after 4000 keys: 25.1 us
 // against 26.5; 37 after 2000: 15.0 against 18.4) and segments win the long ones (8 after 4000: 22.3 -> 14.9;
 // 37 after 12000: 57.2 -> 28.1; 100 after 20000: 89.9 -> 49.8; 500 after 8000: 94.9 -> 74.3; 64/8, 100 after
 // 20000: 106.2 -> 77.9).  Against row blocks of two heads, whose launches mostly take several rounds, several segments
@@ -493,7 +494,7 @@ int plan_shared_segments(int q_len, int kv_span, bool causal, int group, int n_k
         const double us = (segs > 1 ? 10.0 : 4.0) + 0.7 * mb + loop_us;
         if (segs > 1 && rows_gpu_us < 7.5) break;  // the host's time for two launches
         const double gpu_us = std::max(0.4 * us, 1.05 * ((double)(base * segs) / n_cu * (4.0 + loop_us) + 0.3 * mb));
-        const double cost = two_heads ? (segs > 1 ? us / 1.1 : (us + 4.0) / 1.2) : segs > 1 ? us + 4.0 : us;
+        const double cost = two_heads ? (segs > 1 ? us / 1.1 : (us + 4.0) / 1.2) : segs > 1 ? us + 4.0 : us + 0.25;
         if (cost < best_us && gpu_us <= (two_heads ? (segs > 1 ? 0.95 : 0.6) : 1.0) * rows_gpu_us) {
             best_us = cost;
             best = segs;

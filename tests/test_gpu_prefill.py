@@ -713,3 +713,16 @@ def test_loads_of_growing_length():
                 acc.load_kv(k, v, start_pos=first)
                 kr, vr = acc.read_kv(0, first, n)
                 assert np.array_equal(kr, k) and np.array_equal(vr, v)
+
+
+@pytest.mark.parametrize("hq,hkv,d,q_len", [(8, 2, 64, 8), (32, 8, 64, 1), (8, 8, 64, 31), (8, 8, 128, 30), (64, 4, 64, 2)])
+def test_prompts_of_one_key_block_take_row_blocks(hq, hkv, d, q_len):
+    """AUTO for the smallest prompts (one key block, fewer rows than a task): row blocks, against the oracle."""
+    rng = np.random.default_rng(5600 + hq + d + q_len)
+    print(f"[tiny] hq={hq} hkv={hkv} d={d} q_len={q_len}", flush=True)
+    q, k, v = (bf16_normal(rng, (h, q_len, d)) for h in (hq, hkv, hkv))
+    with AttentionAccelerator(n_q_heads=hq, n_kv_heads=hkv, head_dim=d, max_seq_len=64, max_q_len=64) as acc:
+        out, lse = acc.prefill_chunk(q, kv_len=q_len, k_rows=k, v_rows=v, return_lse=True)
+        assert acc.last_prefill_plan() == ("rows", 1)
+    ref, ref_lse = oracle_for(q, k, v, causal=True, q_pos_base=0)
+    check_rows(out, lse, ref, ref_lse)
