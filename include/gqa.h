@@ -101,8 +101,9 @@ extern "C" {
  * that asks for it a second time without a launch of that stream in between); else SHARED -- paired when
  * that grid is exactly one work-group per CU (for instance a causal 2048-row chunk after earlier keys at
  * 32q/8kv on 256 CUs), unpaired when larger.  gqa_last_prefill_plan reports the decomposition a launch took.
- * Launches in several segments under a forced decomposition or segment target share a workspace of their own:
- * the caller orders them among each other (streams, replayed graphs); AUTO's may be in flight beside them. */
+ * Launches in several segments under a forced decomposition or segment target share a workspace of their own,
+ * which these options allocate (a forced decomposition without memory for it takes one segment): the caller
+ * orders them among each other (streams, replayed graphs); AUTO's may be in flight beside them. */
 #define GQA_PREFILL_KERNEL_AUTO   0
 #define GQA_PREFILL_KERNEL_SHARED 1
 #define GQA_PREFILL_KERNEL_ROWS   2
